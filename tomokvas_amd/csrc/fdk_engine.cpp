@@ -295,6 +295,13 @@ double out_scale(const fdk_ctx *c, int dtype)
     return (double)(c->g.dbeta * (1.0f / (float)c->p));
 }
 
+// The per-projection maxima that the filter leaves for the pack: only FP16
+// storage scales by them, so the other storage types filter without them.
+unsigned *pack_maxabs(const fdk_ctx *c)
+{
+    return c->storage == FDK_F16 || c->storage == FDK_F16_PACKED ? c->d_maxabs : nullptr;
+}
+
 int stage_filter(fdk_ctx *c, int dtype, const void *in, void *out, int nang, int weight,
                  int adjoint, unsigned *maxabs, hipStream_t st)
 {
@@ -929,14 +936,15 @@ int fdk_calculate_reconstruction(fdk_ctx *c, fdk_get_block_fn get_block, void *u
     if ((rc = after_caller_work(c))) return rc;
     const tkv::Geometry &g = c->g;
     hipStream_t st = c->stream;
-    if ((rc = tkv::launch_zero_u32(c->d_maxabs, g.Nang, st))) return rc;
+    unsigned *const maxabs = pack_maxabs(c);
+    if (maxabs && (rc = tkv::launch_zero_u32(maxabs, g.Nang, st))) return rc;
     TKV_HIP(hipEventRecord(c->ev[0], st));
     // cosine weight fused into the row filter (kernel.cu:807-808)
-    if ((rc = stage_filter(c, FDK_F32, c->d_sino, c->d_filt, g.Nang, 1, 0, c->d_maxabs, st)))
+    if ((rc = stage_filter(c, FDK_F32, c->d_sino, c->d_filt, g.Nang, 1, 0, maxabs, st)))
         return rc;
     TKV_HIP(hipEventRecord(c->ev[1], st));
     if ((rc = tkv::launch_pack(FDK_F32, c->d_filt, g.Nu, g.Nv, g.Nang, tkv::stack_pitch(g.Nu),
-                               c->d_maxabs, c->storage, c->d_stack, c->d_scales, st)))
+                               maxabs, c->storage, c->d_stack, c->d_scales, st)))
         return rc;
     TKV_HIP(hipEventRecord(c->ev[2], st));
     if (!get_block) {
@@ -1019,7 +1027,8 @@ int fdk_reconstruct_host(fdk_ctx *c, const float *host_sino, fdk_get_block_fn ge
         return FDK_OK;
     };
     hipStream_t ps = c->prep_stream;
-    if ((rc = tkv::launch_zero_u32(c->d_maxabs, g.Nang, ps))) return rc;
+    unsigned *const maxabs = pack_maxabs(c);
+    if (maxabs && (rc = tkv::launch_zero_u32(maxabs, g.Nang, ps))) return rc;
     TKV_HIP(hipEventRecord(c->ev[0], cs));
     if ((rc = upload(0))) return rc;
     for (int k = 0; k < K; ++k) {
@@ -1031,9 +1040,10 @@ int fdk_reconstruct_host(fdk_ctx *c, const float *host_sino, fdk_get_block_fn ge
         // so they can run while the previous chunk is backprojected; its
         // backprojection on the compute stream once they are done
         TKV_HIP(hipStreamWaitEvent(ps, c->ev_up[k & 1], 0));
-        if ((rc = stage_filter(c, FDK_F32, in, filt, nc, 1, 0, c->d_maxabs + a0, ps)) ||
-            (rc = tkv::launch_pack(FDK_F32, filt, g.Nu, g.Nv, nc, pitch, c->d_maxabs + a0,
-                                   c->storage, stack, scales, ps)))
+        unsigned *const mx = maxabs ? maxabs + a0 : nullptr;
+        if ((rc = stage_filter(c, FDK_F32, in, filt, nc, 1, 0, mx, ps)) ||
+            (rc = tkv::launch_pack(FDK_F32, filt, g.Nu, g.Nv, nc, pitch, mx, c->storage, stack,
+                                   scales, ps)))
             break;
         TKV_HIP(hipEventRecord(c->ev_f[k & 1], ps));
         TKV_HIP(hipStreamWaitEvent(st, c->ev_f[k & 1], 0));

@@ -130,6 +130,15 @@ __device__ __forceinline__ R group_max(R m, int width)
 __device__ __forceinline__ unsigned float_bits_abs(float m) { return __float_as_uint(m); }
 __device__ __forceinline__ unsigned float_bits_abs(double m) { return __float_as_uint((float)m); }
 
+// *p = max(*p, m) over the whole grid.  Atomics on one cache line run one after
+// another, and a stack of n projections has only n addresses, so the value is
+// read first and the atomic issued only to raise it: *p never falls, so a
+// value that is out of date only costs an atomic too many.
+__device__ __forceinline__ void raise_max(unsigned *p, unsigned m)
+{
+    if (m > __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(p, m);
+}
+
 // ---------------------------------------------------------------- radix-16 row filter
 // Mixed-radix Stockham plan: passes of radix RMAX (16, or 8), with the one
 // smaller pass that log2(p) mod log2(RMAX) requires placed second, so the first
@@ -485,8 +494,8 @@ __global__ void __launch_bounds__(PL::BLOCK) __attribute__((amdgpu_waves_per_eu(
         mB = group_max(mB, PL::TPT);
         bool leader = (PL::TPT >= 64) ? ((tid & 63) == 0) : (t == 0);
         if (leader) {
-            if (hasA) atomicMax(&maxabs[rA % nang], float_bits_abs(mA));
-            if (hasB) atomicMax(&maxabs[rB % nang], float_bits_abs(mB));
+            if (hasA) raise_max(&maxabs[rA % nang], float_bits_abs(mA));
+            if (hasB) raise_max(&maxabs[rB % nang], float_bits_abs(mB));
         }
     }
 }
