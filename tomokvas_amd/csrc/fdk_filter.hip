@@ -490,12 +490,26 @@ __global__ void __launch_bounds__(PL::BLOCK) __attribute__((amdgpu_waves_per_eu(
         }
     }
     if (maxabs) {
+        // the workgroup's rows are 2 NT consecutive ones, so their maxima lie side
+        // by side: collected through LDS and raised by the lanes of one wave,
+        // one request to the cache line instead of two per wave
+        constexpr int PARTS = PL::TPT >= 64 ? PL::TPT / 64 : 1;   // waves of a transform
+        __shared__ unsigned part[2 * PL::NT * PARTS];
         mA = group_max(mA, PL::TPT);
         mB = group_max(mB, PL::TPT);
-        bool leader = (PL::TPT >= 64) ? ((tid & 63) == 0) : (t == 0);
-        if (leader) {
-            if (hasA) raise_max(&maxabs[rA % nang], float_bits_abs(mA));
-            if (hasB) raise_max(&maxabs[rB % nang], float_bits_abs(mB));
+        if (PL::TPT >= 64 ? (tid & 63) == 0 : t == 0) {
+            const int w = PL::TPT >= 64 ? (t >> 6) : 0;
+            part[2 * (f * PARTS + w)] = float_bits_abs(mA);
+            part[2 * (f * PARTS + w) + 1] = float_bits_abs(mB);
+        }
+        __syncthreads();
+        for (int i = tid; i < 2 * PL::NT; i += PL::BLOCK) {
+            const long long r = 2 * (long long)blockIdx.x * PL::NT + i;
+            unsigned m = 0;
+#pragma unroll
+            for (int w = 0; w < PARTS; ++w)
+                m = max(m, part[2 * ((i >> 1) * PARTS + w) + (i & 1)]);
+            if (r < rows) raise_max(&maxabs[r % nang], m);
         }
     }
 }
