@@ -21,11 +21,12 @@ constexpr int BOX_ALIGN = 4;   // box columns start on a multiple of 4 samples
 // that the block's bilinear taps can touch, widened by 2 samples on each side
 // for the rounding of the per-column values (the columns evaluate the same
 // float expressions as the corners); bw == 0: the block misses the detector;
-// bw < 0: go through HBM directly (box beyond the LDS tile, or a block corner
-// near or behind the source plane, where U is not monotone over the block).
+// bw < 0: go through HBM directly (box beyond the LDS tile of box_w columns and
+// box_h rows, or a block corner near or behind the source plane, where U is not
+// monotone over the block).
 __device__ inline int4 footprint(float c, float s, float x0, float x1, float y0, float y1,
                                  float azlo, float azhi, float cX, float cZ, float D, int Nu,
-                                 int Nv, int box_h)
+                                 int Nv, int box_h, int box_w = BOX_W)
 {
     float umin = 3.0e38f, umax = -3.0e38f, Umin = 3.0e38f, Umax = -3.0e38f;
     bool ok = true;
@@ -58,7 +59,7 @@ __device__ inline int4 footprint(float c, float s, float x0, float x1, float y0,
     const int bv1 = min((int)fv1 + 3, Nv - 1);
     const int bw = bu1 - bu0 + 1, bh = bv1 - bv0 + 1;
     if (bw <= 0 || bh <= 0) return make_int4(0, 0, 0, 0);
-    if (bw >= BOX_W || bh >= box_h) return make_int4(0, 0, -1, 0);
+    if (bw >= box_w || bh >= box_h) return make_int4(0, 0, -1, 0);
     // bit 16 of the width: every sample row of the block lies inside
     // [0.02, Nv-1.02] (the per-column rows differ from the corner bounds by
     // rounding only), so the gathers need no range test
