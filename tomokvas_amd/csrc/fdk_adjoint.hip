@@ -348,7 +348,7 @@ __global__ void __launch_bounds__(64 * FP_WAVES) fp_lds_kernel(FPArgs<float> a)
             // splat into the LDS box; taps with zero weight past the
             // detector's last row or column land inside the box and are
             // dropped at the flush
-            const bool inner = bw & 0x10000;
+            const bool inner = bw & BOX_INNER_V;
             char *lds = (char *)cur;
             // LDS byte offset of the column's sample in detector row 0; the
             // weights in units of 1/fxs

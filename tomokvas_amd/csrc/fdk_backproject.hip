@@ -371,10 +371,9 @@ struct BoxStage {
         const int nrec = (rows + 1) * (int)row_bytes - bu0 * ST::BYTES;
         const __amdgpu_buffer_rsrc_t rsrc =
             __builtin_amdgcn_make_buffer_rsrc((void *)base, (short)0, nrec, 0x00020000);
-        const uint32_t off0 = (threadIdx.x >> 4) * row_bytes + (threadIdx.x & 15) * 4 * ST::BYTES;
+        int off = (int)((threadIdx.x >> 4) * row_bytes + (threadIdx.x & 15) * 4 * ST::BYTES);
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int off = (int)(off0 + (uint32_t)(16 * i) * row_bytes);
+        for (int i = 0; i < PER; ++i, off += (int)(16 * row_bytes)) {
             if constexpr (ST::BYTES == 4) {
                 const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0);
                 raw[i] = make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]),
@@ -427,6 +426,19 @@ __device__ __forceinline__ float uniform_load(const float *p)
     return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(*p)));
 }
 
+// n / d correctly rounded (Markstein 1990: a Newton step on the reciprocal, two
+// residual corrections of the quotient) for normal n, d and quotient: without
+// the exponent scaling and special cases of the general division, 9
+// instructions instead of 13.  The staged angles have d = D - S > D/100.
+__device__ __forceinline__ float div_normal(float n, float d)
+{
+    float r = __builtin_amdgcn_rcpf(d);
+    r = fmaf(fmaf(-d, r, 1.f), r, r);
+    float q = n * r;
+    q = fmaf(fmaf(-d, q, n), r, q);
+    return fmaf(fmaf(-d, q, n), r, q);
+}
+
 // ---- the backprojector --------------------------------------------------------------
 template <typename S, int ZR, int LB>
 __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
@@ -436,13 +448,16 @@ __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
     constexpr bool STAGED = ST::STAGED;
     constexpr int BOX_H = box_rows<ZR>();
     constexpr int P = ST::P;
+    constexpr int INNER_U = 1 << 30;   // flag beside an angle's index
     static_assert(P >= BOX_W && P % 4 == 0, "box pitch");
     __shared__ float boxmem[STAGED ? P * BOX_H : 1];
-    // per group of 64 angles, in two slots (groups g and g+1): the footprints,
-    // the group's angle order (inner angles from the front, edge angles from
-    // the back) and the two counts; and whether any angle is left to pass 2
-    __shared__ int4 boxes[STAGED ? 128 : 1];
-    __shared__ unsigned char order[STAGED ? 128 : 1];
+    // per group of 64 angles, in two slots (groups g and g+1): the staged angles,
+    // inner ones first (first column and last row of the footprint, its first
+    // row, the angle's index, cos), with their sin and scale; the number of inner
+    // and of all staged angles; and whether any angle is left to pass 2.  (Kept
+    // within 3 KiB, so that five FP16 workgroups fit a CU.)
+    __shared__ int4 ebox[STAGED ? 128 : 1];
+    __shared__ float2 ess[STAGED ? 128 : 1];
     __shared__ int counts[4];
     __shared__ int hbm_flag;
 
@@ -509,40 +524,45 @@ __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
         // range tests) and edge ones; each kind runs in a loop of its own, so
         // the accumulators never pass a branch merge (which costs a copy of
         // all of them per angle).  Angles missing the detector are dropped;
-        // those whose box exceeds the tile are left to pass 2.
+        // those whose box exceeds the tile are left to pass 2.  A staged angle's
+        // cos, sin and scale come from LDS, so that nothing of its set-up waits
+        // for memory.
         bool need_hbm = !STAGED;
         if constexpr (STAGED) {
-            auto boxes_of_group = [&](int g) {
+            const bool any_in = __any(inside), all_in = __all(inside);
+            auto angles_of_group = [&](int g) {
                 if (wave != 0) return;
                 const int bb = g * 64 + lane, slot = g & 1;
                 int4 q = make_int4(0, 0, 0, 0);
-                if (bb < a.nang)
-                    q = footprint(a.ang[2 * bb], a.ang[2 * bb + 1], cx0, cx1, cy0, cy1, azlo, azhi,
-                                  a.cX, a.cZ, a.D, a.Nu, a.Nv, BOX_H);
-                boxes[slot * 64 + lane] = q;
-                const bool inner = q.z > 0 && (q.z & 0x10000);
-                const bool edge = q.z > 0 && !(q.z & 0x10000);
-                const uint64_t mi = __ballot(inner), me = __ballot(edge);
+                float c = 0.f, s = 0.f;
+                if (bb < a.nang) {
+                    c = a.ang[2 * bb];
+                    s = a.ang[2 * bb + 1];
+                    q = footprint(c, s, cx0, cx1, cy0, cy1, azlo, azhi, a.cX, a.cZ, a.D, a.Nu,
+                                  a.Nv, BOX_H);
+                }
+                const bool staged = q.z > 0, inner = staged && (q.z & BOX_INNER_V);
+                const uint64_t mi = __ballot(inner), me = __ballot(staged && !inner);
                 const uint64_t mh = __ballot(q.z < 0);
-                // rank among the lanes below of the same kind
-                const int ri = __builtin_amdgcn_mbcnt_hi((unsigned)(mi >> 32),
-                                                         __builtin_amdgcn_mbcnt_lo((unsigned)mi, 0));
-                const int re = __builtin_amdgcn_mbcnt_hi((unsigned)(me >> 32),
-                                                         __builtin_amdgcn_mbcnt_lo((unsigned)me, 0));
-                if (inner) order[slot * 64 + ri] = (unsigned char)lane;
-                if (edge) order[slot * 64 + 63 - re] = (unsigned char)lane;
+                // rank among the lanes below of the same kind, inner ones first
+                const uint64_t mk = inner ? mi : me;
+                const int rank =
+                    __builtin_amdgcn_mbcnt_hi((unsigned)(mk >> 32),
+                                              __builtin_amdgcn_mbcnt_lo((unsigned)mk, 0)) +
+                    (inner ? 0 : __popcll(mi));
+                if (staged) {
+                    // the index with a flag: every tap column lies on the detector
+                    // (columns are below 8192, a box has at most 127 rows)
+                    ebox[slot * 64 + rank] =
+                        make_int4(q.x | q.w << 16, q.y, bb | (q.z & BOX_INNER_U ? INNER_U : 0),
+                                  __float_as_int(c));
+                    ess[slot * 64 + rank] = make_float2(s, a.scales[bb] * wnorm);
+                }
                 if (lane == 0) {
                     counts[2 * slot] = __popcll(mi);
-                    counts[2 * slot + 1] = __popcll(me);
+                    counts[2 * slot + 1] = __popcll(mi) + __popcll(me);
                     if (mh) hbm_flag = 1;
                 }
-            };
-            auto uniform_box = [&](int slot, int i) {
-                const int4 q = boxes[slot * 64 + i];
-                return make_int4(__builtin_amdgcn_readfirstlane(q.x),
-                                 __builtin_amdgcn_readfirstlane(q.y),
-                                 __builtin_amdgcn_readfirstlane(q.z),
-                                 __builtin_amdgcn_readfirstlane(q.w));
             };
             auto uniform_int = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
             // the tile starts finite: rows of a box past its last 16-row block
@@ -550,99 +570,96 @@ __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
             for (int i = threadIdx.x; i < P * BOX_H; i += 256) boxmem[i] = 0.f;
             if (threadIdx.x == 0) hbm_flag = 0;
             __syncthreads();
-            boxes_of_group(0);
-            boxes_of_group(1);
+            angles_of_group(0);
+            angles_of_group(1);
             __syncthreads();
             BoxStage<S, BOX_H> stage;
-            auto issue = [&](int b, int4 q) {
-                stage.issue(a.stack + (size_t)b * a.angle_bytes, q.x, q.y, q.w, a.row_bytes, a.Nv);
+            // the box being loaded: first column, first row, last row, index
+            int bu0 = 0, bv0 = 0, bh = -1, bi = 0;
+            auto issue = [&](const int4 &e) {
+                const int uh = uniform_int(e.x);
+                bu0 = uh & 0xffff;
+                bh = uh >> 16;
+                bv0 = uniform_int(e.y);
+                bi = uniform_int(e.z);
+                stage.issue(a.stack + (size_t)(bi & ~INNER_U) * a.angle_bytes, bu0, bv0, bh,
+                            a.row_bytes, a.Nv);
             };
-            // column weights and LDS offsets of one staged angle, then its gathers
-            auto gather_angle = [&](auto fast_tag, int b, int4 bx) {
+            // column weights and LDS offsets of the staged angle, then its gathers
+            auto gather_angle = [&](auto fast_tag, int qu, int qv, bool inner_u, float wc, float ws,
+                                    float wscale) {
                 constexpr bool FAST = decltype(fast_tag)::value;
-                const R c = a.ang[2 * b], s = a.ang[2 * b + 1];
                 // the reference's S, T, U and u with nvcc's contractions; the
                 // packed-FP16 path, whose error is set by its FP16 weights,
                 // takes U from the hardware reciprocal instead of the IEEE
                 // quotient
-                const R Sx = rfma(aX, c, aY * s);
-                const R T = rfma(aY, c, -(aX * s));
+                const R Sx = rfma(aX, wc, aY * ws);
+                const R T = rfma(aY, wc, -(aX * ws));
                 R U;
                 if constexpr (PACKED)
                     U = a.D * __builtin_amdgcn_rcpf(a.D - Sx);
                 else
-                    U = a.D / (a.D - Sx);
+                    U = div_normal(a.D, a.D - Sx);
                 const R u = rfma(T, U, a.cX);
-                const bool act = inside && u >= (R)0 && u <= a.umax;
                 const R fu = rfract(u);
-                const int iu = act ? (int)u : 0;            // u >= 0: trunc = floor
-                const R W = act ? U * U * (a.scales[b] * wnorm) : (R)0;
+                int iu = (int)u;                            // u >= 0: trunc = floor
+                R W = U * U * wscale;
+                R Uv = U, cz = a.cZ;
+                // inactive lanes get weight 0 and sit at v = bv0, column 0; no
+                // lane is inactive when every column of the wave lies in the
+                // cylinder and every tap column on the detector
+                if (!(all_in && inner_u)) {
+                    const bool act = inside && u >= (R)0 && u <= a.umax;
+                    iu = act ? iu : qu;
+                    W = act ? W : (R)0;
+                    Uv = act ? Uv : (R)0;
+                    cz = act ? cz : (R)qv;
+                }
                 const R wu1 = W * fu, wu0 = W - wu1;
                 half2_t wuh = {0, 0};
                 if constexpr (PACKED) wuh = half2_t{(_Float16)wu0, (_Float16)wu1};
                 // LDS byte offset of sample (row iv, column iu) is
-                // iv*4*P + colb; inactive lanes sit at v = bv0, offset 0
-                const int colb = (act ? (iu - bx.x) * 4 : 0) - bx.y * (4 * P);
-                const R Uv = act ? U : (R)0;
-                const R cz = act ? a.cZ : (R)bx.y;
+                // iv*4*P + colb
+                const int colb = iu * 4 - (qu * 4 + qv * (4 * P));
                 gather_run<FAST, ST::PAIRS, ST::MIX, ZR, LB, P>(acc, az, boxmem, Uv, cz, colb,
                                                                 wu0, wu1, wuh, a.vmax, a.one);
             };
             using fast_t = std::integral_constant<bool, true>;
             using edge_t = std::integral_constant<bool, false>;
             const int ngroups = (a.nang + 63) >> 6;
-            int pf = -1;   // angle whose box the stage registers are loading
+            bool loading = false;   // this group's first box is already on its way
             for (int g = 0; g < ngroups; ++g) {
-                const int slot = g & 1, g0 = g * 64;
+                const int slot = g & 1;
                 if (g > 0) {
                     // the slot of group g-1 is free once every wave is here
                     __syncthreads();
-                    boxes_of_group(g + 1);
+                    angles_of_group(g + 1);
                     __syncthreads();
                 }
-                // edge angles: loaded and gathered one at a time
-                const int ne = uniform_int(counts[2 * slot + 1]);
-                for (int j = 0; j < ne; ++j) {
-                    const int i = uniform_int(order[slot * 64 + 63 - j]);
-                    const int4 bx = uniform_box(slot, i);
-                    issue(g0 + i, bx);
-                    __syncthreads();   // every wave is done with the previous box
-                    stage.commit(boxmem, bx.w);
-                    __syncthreads();
-                    gather_angle(edge_t{}, g0 + i, bx);
-                }
-                // inner angles: the next one's box is loaded while one is gathered
-                const int ni = uniform_int(counts[2 * slot]);
-                if (ni > 0) {
-                    const int i = uniform_int(order[slot * 64]);
-                    if (pf != g0 + i) issue(g0 + i, uniform_box(slot, i));
-                }
-                pf = -1;
-                for (int j = 0; j < ni; ++j) {
-                    const int i = uniform_int(order[slot * 64 + j]);
-                    const int4 bx = uniform_box(slot, i);
-                    __syncthreads();   // every wave is done with the previous box
-                    stage.commit(boxmem, bx.w);
-                    __syncthreads();
-                    // the next inner angle: this group's, else the next group's
-                    // first when that group has no edge angles (whose loads
-                    // would take the stage registers)
-                    int nb = -1;
-                    int4 nq = make_int4(0, 0, 0, -1);   // none: an empty range, zeros
-                    if (j + 1 < ni) {
-                        const int k = uniform_int(order[slot * 64 + j + 1]);
-                        nb = g0 + k;
-                        nq = uniform_box(slot, k);
-                    } else if (g + 1 < ngroups && uniform_int(counts[2 * (slot ^ 1) + 1]) == 0 &&
-                               uniform_int(counts[2 * (slot ^ 1)]) > 0) {
-                        const int k = uniform_int(order[(slot ^ 1) * 64]);
-                        nb = g0 + 64 + k;
-                        nq = uniform_box(slot ^ 1, k);
+                const int ni = uniform_int(counts[2 * slot]), n = uniform_int(counts[2 * slot + 1]);
+                const int n1 = uniform_int(counts[2 * (slot ^ 1) + 1]);
+                if (!loading && n > 0) issue(ebox[slot * 64]);
+                loading = n > 0 && g + 1 < ngroups && n1 > 0;
+                // entries [e0, e1); while one is gathered the next one's box is
+                // loaded (the next group's first after the last)
+                auto run = [&](auto fast_tag, int e0, int e1) {
+                    for (int j = e0; j < e1; ++j) {
+                        const int qu = bu0, qv = bv0, qh = bh;
+                        const bool inner_u = bi & INNER_U;
+                        const int at = j + 1 < n ? slot * 64 + j + 1 : (slot ^ 1) * 64;
+                        const bool more = j + 1 < n || loading;
+                        const int4 e = ebox[at];            // (read, not used, if no more)
+                        const float wc = __int_as_float(ebox[slot * 64 + j].w);
+                        const float2 ss = ess[slot * 64 + j];
+                        __syncthreads();   // every wave is done with the previous box
+                        stage.commit(boxmem, qh);
+                        __syncthreads();
+                        if (more) issue(e);
+                        if (any_in) gather_angle(fast_tag, qu, qv, inner_u, wc, ss.x, ss.y);
                     }
-                    issue(nb >= 0 ? nb : 0, nq);
-                    pf = nb;
-                    gather_angle(fast_t{}, g0 + i, bx);
-                }
+                };
+                run(fast_t{}, 0, ni);
+                run(edge_t{}, ni, n);
             }
             need_hbm = uniform_int(hbm_flag) != 0;
         }

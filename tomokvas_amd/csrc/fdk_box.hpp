@@ -14,9 +14,12 @@ constexpr int BOX_W = 64;
 template <int ZR>
 constexpr int box_rows() { return ZR > 32 ? 128 : ZR > 24 ? 96 : ZR > 16 ? 80 : 64; }
 constexpr int BOX_ALIGN = 4;   // box columns start on a multiple of 4 samples
+// flags beside the box's width: every tap row, or column, of the block lies on
+// the detector
+constexpr int BOX_INNER_V = 0x10000, BOX_INNER_U = 0x20000;
 
 // ---- footprint box of a block for one angle ----------------------------------------
-// Returns (bu0, bv0, bw | inner << 16, bh): the detector samples
+// Returns (bu0, bv0, bw | flags, bh): the detector samples
 // [bu0, bu0+bw) x [bv0, bv0+bh)
 // that the block's bilinear taps can touch, widened by 2 samples on each side
 // for the rounding of the per-column values (the columns evaluate the same
@@ -60,11 +63,12 @@ __device__ inline int4 footprint(float c, float s, float x0, float x1, float y0,
     const int bw = bu1 - bu0 + 1, bh = bv1 - bv0 + 1;
     if (bw <= 0 || bh <= 0) return make_int4(0, 0, 0, 0);
     if (bw >= box_w || bh >= box_h) return make_int4(0, 0, -1, 0);
-    // bit 16 of the width: every sample row of the block lies inside
-    // [0.02, Nv-1.02] (the per-column rows differ from the corner bounds by
-    // rounding only), so the gathers need no range test
+    // flags: every sample row of the block lies inside [0.02, Nv-1.02], every
+    // column inside [0.02, Nu-1.02] (the per-column values differ from the corner
+    // bounds by rounding only), so the gathers need no range test
     const bool inner = vlo >= 0.02f && vhi <= (float)(Nv - 1) - 0.02f;
-    return make_int4(bu0, bv0, bw | (inner ? 0x10000 : 0), bh);
+    const bool inner_u = umin >= 0.02f && umax <= (float)(Nu - 1) - 0.02f;
+    return make_int4(bu0, bv0, bw | (inner ? BOX_INNER_V : 0) | (inner_u ? BOX_INNER_U : 0), bh);
 }
 
 }  // namespace tkv
