@@ -110,3 +110,36 @@ def test_adjoint_at_tiny_and_huge_values(torch):
     for s in (2.0 ** -90, 2.0 ** 90):
         y = st.forward_project(torch.from_numpy(x * np.float32(s)).cuda()).double().cpu().numpy()
         assert O.rel_rmse(y / s, one) <= 1e-6
+
+
+# box heights from 16 rows to the limit and beyond it (gathered from HBM): small
+# and large voxels, a source close to the object (U up to 2.5), a tall volume
+# whose top and bottom runs leave the detector
+BP_CASES = {
+    "fine": dict(Nu=40, Nv=36, Nang=9, Nx=60, Ny=44, Nz=70, D=300.0, scale=0.4),
+    "coarse": dict(Nu=90, Nv=100, Nang=9, Nx=40, Ny=37, Nz=40, D=500.0, scale=2.3),
+    "near": dict(Nu=64, Nv=64, Nang=70, Nx=50, Ny=50, Nz=50, D=54.0, scale=1.1),
+    "tall": dict(Nu=64, Nv=24, Nang=130, Nx=48, Ny=48, Nz=99, D=200.0, scale=1.25, cX=29.5),
+}
+
+
+@pytest.mark.parametrize("case", list(BP_CASES))
+@pytest.mark.parametrize("store", [_lib.F32, _lib.F16, _lib.BF16])
+def test_backprojection_boxes(torch, case, store):
+    """Against the FP32 mirror's backprojection of the decoded samples: positions
+    and weights are the same bits, the sums are rounded in another order."""
+    g = scan(**BP_CASES[case], tau=0.1)
+    st = stages(g)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    d = torch.randn(st.sino_shape(), device="cuda", generator=gen)
+    m = d.abs().amax(dim=(0, 2)).view(torch.int32)
+    say(f"backprojection {case}, storage {store}")
+    stack, scales = st.pack(d, store, m)
+    got = st.backproject(stack, store, scales).cpu().numpy()
+    # the stored samples [Nang][Nv][pitch], decoded
+    dt = {_lib.F32: torch.float32, _lib.F16: torch.float16, _lib.BF16: torch.bfloat16}[store]
+    per = st.stack_bytes(store, 1) - st.stack_bytes(store, 0)
+    q = stack[:per * g.Nang].view(dt).view(g.Nang, g.Nv, -1)[:, :, :g.Nu].float()
+    dec = (q * scales[:, None, None]).transpose(0, 1).contiguous()
+    ref = O.backproject(ogeom(g), dec.cpu().numpy())
+    assert O.rel_rmse(got, ref) <= 1e-6

@@ -18,15 +18,16 @@
 //    voxel-updates instead of four taps per update;
 //  * the stored stack is plain and angle-major ([beta][v][pitch]) in the
 //    storage type: FP32, FP16 with a per-projection scale, or BF16; FP16 and
-//    BF16 halve the staging bytes.  FP32 and BF16 boxes hold FP32 samples.
-//    FP16 boxes keep FP16 sample pairs (q[c], q[c+1]) per 32-bit word, which
-//    halves the LDS bytes of a gather; the FP16 path (FDK_F16) widens them
-//    inside mixed-precision FMAs (v_fma_mix_f32: FP16 samples, FP32 fraction,
-//    differences and weights, FP32 result), so for every storage type the
-//    interpolation weights, lerps and accumulation are FP32 and the FP16
-//    volume is the FP32 arithmetic on the decoded samples.  FDK_F16_PACKED
-//    (opt-in) instead lerps in packed FP16 and weights with v_dot2 (FP16
-//    fraction and column weights): faster, outside that precision form;
+//    BF16 halve the staging bytes.  The box in LDS holds FP32 samples, widened
+//    exactly when they are staged, so for every storage type the interpolation
+//    weights, lerps and accumulation are FP32 and a low-precision volume is the
+//    FP32 arithmetic on the decoded samples.  (FP16 pairs in the box, widened by
+//    mixed-precision FMAs, halve the LDS reads, but those FMAs issue at 1.1
+//    cycles per wave instruction and CU where plain FP32 arithmetic on vector
+//    registers takes 0.66: 38.9 against 37.6 ms for 512^3 from 900 x 1024^2.)
+//    FDK_F16_PACKED (opt-in) keeps FP16 pairs (q[c], q[c+1]) per 32-bit word,
+//    lerps in packed FP16 and weights with v_dot2 (FP16 fraction and column
+//    weights): faster, outside the precision form;
 //  * z-runs that project entirely inside the detector for every active lane of
 //    a wave (the common case) skip the per-slice range test;
 //  * workgroup ids are remapped so the workgroups an XCD runs together cover a
@@ -40,6 +41,7 @@
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
+#include <cmath>
 #include <type_traits>
 
 // Tuning knobs (defaults chosen by measurement on MI355X, 1024^3 from
@@ -49,10 +51,10 @@
 //   TKV_BP_LB                      LDS gathers per lane issued together
 //   TKV_BP_GROUP_FENCE             1: no instruction moves between groups of
 //                                  LB gathers
-//   TKV_BP_BOXP_F32 / _F16 / _BF16 LDS row pitch of the staged box in 32-bit
+//   TKV_BP_BOXP_F32 / _F16P        LDS row pitch of the staged box in 32-bit
 //                                  words (>= 64, multiple of 4): rows of one
-//                                  column fall in different banks (the FP16
-//                                  pitch serves FDK_F16 and FDK_F16_PACKED)
+//                                  column fall in different banks (FP32 samples;
+//                                  FP16 pairs)
 #ifndef TKV_BP_ZR_F32
 #define TKV_BP_ZR_F32 24
 #endif
@@ -72,14 +74,11 @@
 #ifndef TKV_BP_GROUP_FENCE
 #define TKV_BP_GROUP_FENCE 1
 #endif
-#ifndef TKV_BP_BOXP_F16
-#define TKV_BP_BOXP_F16 72
-#endif
 #ifndef TKV_BP_BOXP_F32
 #define TKV_BP_BOXP_F32 80
 #endif
-#ifndef TKV_BP_BOXP_BF16
-#define TKV_BP_BOXP_BF16 80
+#ifndef TKV_BP_BOXP_F16P
+#define TKV_BP_BOXP_F16P 72
 #endif
 
 namespace tkv {
@@ -102,15 +101,15 @@ struct BPArgs {
     R *vol;
     int Nx, Ny, Nz, Nu, Nv, nang;
     R cX, cZ, D, umax, vmax, out_scale;
-    float one;                    // 1.0 (a run-time value: see gather_mix)
     double maskR2;
     int accumulate;
     int tiles_x, tiles_xy, nblocks;
+    int box_h;                    // rows of the LDS box, a multiple of 16
 };
 
 // ---- storage types ----------------------------------------------------------------
-// PAIRS: the LDS box holds FP16 sample pairs; MIX: they are interpolated with
-// FP32 fractions and weights in mixed-precision FMAs (else packed FP16)
+// PAIRS: the LDS box holds FP16 sample pairs, interpolated in packed FP16 (else
+// FP32 samples)
 struct st_f32;
 struct st_f16;
 struct st_bf16;
@@ -126,7 +125,6 @@ struct Store<st_f32> {
     static constexpr int ZR = TKV_BP_ZR_F32;
     static constexpr int P = TKV_BP_BOXP_F32;
     static constexpr bool PAIRS = false;
-    static constexpr bool MIX = false;
     static __device__ __forceinline__ float get(const char *p) { return *(const float *)p; }
     static __device__ __forceinline__ float half(unsigned, int) { return 0.f; }
 };
@@ -136,9 +134,8 @@ struct Store<st_f16> {
     static constexpr int BYTES = 2;
     static constexpr bool STAGED = true;
     static constexpr int ZR = TKV_BP_ZR_F16;
-    static constexpr int P = TKV_BP_BOXP_F16;
-    static constexpr bool PAIRS = true;
-    static constexpr bool MIX = true;
+    static constexpr int P = TKV_BP_BOXP_F32;
+    static constexpr bool PAIRS = false;
     static __device__ __forceinline__ float get(const char *p)
     {
         return __half2float(__ushort_as_half(*(const unsigned short *)p));
@@ -154,9 +151,8 @@ struct Store<st_bf16> {
     static constexpr int BYTES = 2;
     static constexpr bool STAGED = true;
     static constexpr int ZR = TKV_BP_ZR_BF16;
-    static constexpr int P = TKV_BP_BOXP_BF16;
+    static constexpr int P = TKV_BP_BOXP_F32;
     static constexpr bool PAIRS = false;
-    static constexpr bool MIX = false;
     static __device__ __forceinline__ float get(const char *p)
     {
         return __uint_as_float((unsigned)(*(const unsigned short *)p) << 16);
@@ -169,7 +165,8 @@ struct Store<st_bf16> {
 template <>
 struct Store<st_f16p> : Store<st_f16> {
     static constexpr int ZR = TKV_BP_ZR_F16P;
-    static constexpr bool MIX = false;
+    static constexpr int P = TKV_BP_BOXP_F16P;
+    static constexpr bool PAIRS = true;
 };
 template <>
 struct Store<st_f64> {
@@ -179,7 +176,6 @@ struct Store<st_f64> {
     static constexpr int ZR = 8;
     static constexpr int P = 64;   // unused: FP64 is gathered from HBM
     static constexpr bool PAIRS = false;
-    static constexpr bool MIX = false;
     static __device__ __forceinline__ double get(const char *p) { return *(const double *)p; }
     static __device__ __forceinline__ float half(unsigned, int) { return 0.f; }
 };
@@ -227,47 +223,6 @@ __device__ __forceinline__ void gather_lds(float *acc, const float *az, const fl
         const float q10 = p0[P], q11 = p0[P + 1];
         c0[k] = fmaf(fv, q10 - q00, q00);
         c1[k] = fmaf(fv, q11 - q01, q01);
-        okk[k] = ok;
-    }
-    // taps outside the detector get zero weight (the staged values are finite)
-#pragma unroll
-    for (int k = 0; k < LB; ++k)
-        acc[k] = fmaf(okk[k] ? wu1 : 0.f, c1[k], fmaf(okk[k] ? wu0 : 0.f, c0[k], acc[k]));
-}
-
-// FP16 pairs in LDS, FP32 interpolation (FDK_F16): word (r, c) holds samples
-// c and c+1 of row r; one ds_read2 fetches both rows of the 2x2
-// neighbourhood.  Each column's difference along v and its lerp are
-// mixed-precision FMAs reading the FP16 halves directly (v_fma_mix_f32: the
-// product is exact and the result rounds once to FP32, so d = q10 - q00 and
-// c = q00 + fv*d equal the FP32 operations on the widened samples); the
-// column weights (FP32, including the projection's scale) accumulate in FP32.
-template <bool FAST, int LB, int P>
-__device__ __forceinline__ void gather_mix(float *acc, const float *az, const float *box,
-                                           float Uv, float cz, int colb, float wu0, float wu1,
-                                           float vmax, float one)
-{
-    const char *lds = (const char *)box;
-    float c0[LB], c1[LB];
-    bool okk[LB];
-#pragma unroll
-    for (int k = 0; k < LB; ++k) {
-        const float v = fmaf(az[k], Uv, cz);
-        const float fv = __builtin_amdgcn_fractf(v);
-        bool ok = true;
-        int off = (int)__umul24((unsigned)(int)v, 4u * P) + colb;   // v >= 0 where used
-        if (!FAST) {
-            ok = v >= 0.f && v <= vmax;
-            off = ok ? off : 0;
-        }
-        const half2_t w0 = *(const half2_t *)(lds + off);          // (q00, q01)
-        const half2_t w1 = *(const half2_t *)(lds + off + 4 * P);  // (q10, q11)
-        // d = q1*one - q0 (one = 1 at run time: an FMA of the widened halves,
-        // which the compiler forms as v_fma_mix_f32), then c = q0 + fv*d
-        const float d0 = fmaf((float)w1.x, one, -(float)w0.x);
-        const float d1 = fmaf((float)w1.y, one, -(float)w0.y);
-        c0[k] = fmaf(fv, d0, (float)w0.x);
-        c1[k] = fmaf(fv, d1, (float)w0.y);
         okk[k] = ok;
     }
     // taps outside the detector get zero weight (the staged values are finite)
@@ -324,17 +279,14 @@ __device__ __forceinline__ void gather_pairs(float *acc, const float *az, const 
 }
 
 // all ZR slices of a thread for one staged angle, LB gathers at a time
-template <bool FAST, bool PAIRS, bool MIX, int ZR, int LB, int P>
+template <bool FAST, bool PAIRS, int ZR, int LB, int P>
 __device__ __forceinline__ void gather_run(float (&acc)[ZR], const float (&az)[ZR],
                                            const float *box, float Uv, float cz, int colb,
-                                           float wu0, float wu1, half2_t wuh, float vmax,
-                                           float one)
+                                           float wu0, float wu1, half2_t wuh, float vmax)
 {
 #pragma unroll
     for (int k0 = 0; k0 < ZR; k0 += LB) {
-        if constexpr (PAIRS && MIX)
-            gather_mix<FAST, LB, P>(acc + k0, az + k0, box, Uv, cz, colb, wu0, wu1, vmax, one);
-        else if constexpr (PAIRS)
+        if constexpr (PAIRS)
             gather_pairs<FAST, LB, P>(acc + k0, az + k0, box, Uv, cz, colb, wuh, vmax);
         else
             gather_lds<FAST, LB, P>(acc + k0, az + k0, box, Uv, cz, colb, wu0, wu1, vmax);
@@ -349,9 +301,9 @@ __device__ __forceinline__ void gather_run(float (&acc)[ZR], const float (&az)[Z
 // projection (the last is the +1 neighbour row; rows past the detector are
 // zero) x columns [bu0, bu0+64) into registers, 4 samples per lane and row,
 // 16 lanes per row (columns past the row end read the stack's zero padding);
-// commit() writes them into the LDS box.  FP32 boxes hold the samples as
-// floats; FP16 pair boxes hold words (q[c], q[c+1]), the 4th word of a lane
-// taking the next lane's first sample (word 63 is never read).
+// commit() writes them into the LDS box, widened to FP32; FP16 pair boxes hold
+// words (q[c], q[c+1]), the 4th word of a lane taking the next lane's first
+// sample (word 63 is never read).
 template <typename S, int ROWS>
 struct BoxStage {
     using ST = Store<S>;
@@ -372,6 +324,9 @@ struct BoxStage {
         const __amdgpu_buffer_rsrc_t rsrc =
             __builtin_amdgcn_make_buffer_rsrc((void *)base, (short)0, nrec, 0x00020000);
         int off = (int)((threadIdx.x >> 4) * row_bytes + (threadIdx.x & 15) * 4 * ST::BYTES);
+        // the packed-FP16 kernel forms the PER offsets anew for every box: held,
+        // they would take it past the 96 registers of five waves per SIMD
+        if constexpr (ST::PAIRS) asm volatile("" : "+v"(off));
 #pragma unroll
         for (int i = 0; i < PER; ++i, off += (int)(16 * row_bytes)) {
             if constexpr (ST::BYTES == 4) {
@@ -450,7 +405,7 @@ __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
     constexpr int P = ST::P;
     constexpr int INNER_U = 1 << 30;   // flag beside an angle's index
     static_assert(P >= BOX_W && P % 4 == 0, "box pitch");
-    __shared__ float boxmem[STAGED ? P * BOX_H : 1];
+    extern __shared__ __align__(16) float boxmem[];   // a.box_h rows of P words
     // per group of 64 angles, in two slots (groups g and g+1): the staged angles,
     // inner ones first (first column and last row of the footprint, its first
     // row, the angle's index, cos), with their sin and scale; the number of inner
@@ -492,7 +447,7 @@ __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
     // packed FP16 carries the column weights in FP16: they are normalised by
     // the largest projection scale (rounded up to a power of two, g), so they
     // stay within [0, U^2], and the sums are multiplied by g at the end
-    constexpr bool PACKED = ST::PAIRS && !ST::MIX;
+    constexpr bool PACKED = ST::PAIRS;
     R wnorm = 1, wback = 1;
     if constexpr (PACKED) {
         float m = 0.f;
@@ -539,7 +494,7 @@ __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
                     c = a.ang[2 * bb];
                     s = a.ang[2 * bb + 1];
                     q = footprint(c, s, cx0, cx1, cy0, cy1, azlo, azhi, a.cX, a.cZ, a.D, a.Nu,
-                                  a.Nv, BOX_H);
+                                  a.Nv, a.box_h);
                 }
                 const bool staged = q.z > 0, inner = staged && (q.z & BOX_INNER_V);
                 const uint64_t mi = __ballot(inner), me = __ballot(staged && !inner);
@@ -567,7 +522,7 @@ __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
             auto uniform_int = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
             // the tile starts finite: rows of a box past its last 16-row block
             // are never written
-            for (int i = threadIdx.x; i < P * BOX_H; i += 256) boxmem[i] = 0.f;
+            for (int i = threadIdx.x; i < P * a.box_h; i += 256) boxmem[i] = 0.f;
             if (threadIdx.x == 0) hbm_flag = 0;
             __syncthreads();
             angles_of_group(0);
@@ -621,8 +576,8 @@ __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
                 // LDS byte offset of sample (row iv, column iu) is
                 // iv*4*P + colb
                 const int colb = iu * 4 - (qu * 4 + qv * (4 * P));
-                gather_run<FAST, ST::PAIRS, ST::MIX, ZR, LB, P>(acc, az, boxmem, Uv, cz, colb,
-                                                                wu0, wu1, wuh, a.vmax, a.one);
+                gather_run<FAST, ST::PAIRS, ZR, LB, P>(acc, az, boxmem, Uv, cz, colb, wu0, wu1,
+                                                       wuh, a.vmax);
             };
             using fast_t = std::integral_constant<bool, true>;
             using edge_t = std::integral_constant<bool, false>;
@@ -671,7 +626,7 @@ __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
             for (int b = 0; b < a.nang; ++b, proj += a.angle_bytes) {
                 if constexpr (STAGED) {
                     const int4 bx = footprint(a.ang[2 * b], a.ang[2 * b + 1], cx0, cx1, cy0, cy1,
-                                              azlo, azhi, a.cX, a.cZ, a.D, a.Nu, a.Nv, BOX_H);
+                                              azlo, azhi, a.cX, a.cZ, a.D, a.Nu, a.Nv, a.box_h);
                     if (bx.z >= 0) continue;
                 }
                 const R c = a.ang[2 * b], s = a.ang[2 * b + 1];
@@ -747,6 +702,23 @@ int sample_bytes_of(int dtype)
     }
 }
 
+// Rows of the LDS box that every block of this geometry fits (footprint() counts
+// a box's rows plus the +1 neighbour and two of margin either side), a multiple
+// of the 16 rows a load covers, at most box_rows: a workgroup takes no more LDS
+// than its geometry needs, which at two samples per voxel leaves room for five
+// workgroups on a CU instead of four (BF16 512^3 from 900 x 1024^2: 37.5 ms
+// with 96 rows, 36.1 with 80).
+template <int ZR>
+static int box_height(const BPLaunch &L)
+{
+    const double reach = std::sqrt(L.maskR2) + 22. * L.scale;   // a tile's far corner
+    const double U = L.D > reach ? L.D / (L.D - reach) : 100.;
+    // U varies over a tile (15 sqrt 2 voxels across) by at most U^2/D per unit of S
+    const double rows = (ZR - 1) * L.scale * U + L.az_max * 21.3 * L.scale * U * U / L.D + 8.;
+    const int most = box_rows<ZR>();
+    return rows >= most ? most : ((int)rows + 16) / 16 * 16;
+}
+
 template <typename S>
 static int launch_bp_t(const BPLaunch &L, hipStream_t st)
 {
@@ -778,7 +750,6 @@ static int launch_bp_t(const BPLaunch &L, hipStream_t st)
     a.umax = (R)(L.Nu - 1);
     a.vmax = (R)(L.Nv - 1);
     a.out_scale = (R)L.out_scale;
-    a.one = 1.0f;
     a.maskR2 = L.maskR2;
     a.accumulate = L.accumulate;
     a.tiles_x = (L.Nx + 15) / 16;
@@ -788,8 +759,9 @@ static int launch_bp_t(const BPLaunch &L, hipStream_t st)
     if (nb == 0) return FDK_OK;
     if (!grid_fits(nb, 256)) return fail(FDK_ERR_UNSUPPORTED, "backproject: volume too large");
     a.nblocks = (int)nb;
+    a.box_h = Store<S>::STAGED ? box_height<ZR>(L) : 0;
     hipLaunchKernelGGL((bp_kernel<S, ZR, (ZR < TKV_BP_LB ? ZR : TKV_BP_LB)>), dim3((unsigned)nb),
-                       dim3(256), 0, st, a);
+                       dim3(256), sizeof(float) * Store<S>::P * a.box_h, st, a);
     TKV_HIP(hipGetLastError());
     return FDK_OK;
 }

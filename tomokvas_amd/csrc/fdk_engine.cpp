@@ -353,6 +353,8 @@ int stage_backproject(fdk_ctx *c, int store_dtype, const void *stack, const void
     L.D = c->g.D;
     L.out_scale = out_scale(c, store_dtype);
     L.maskR2 = 0.25 * (double)c->g.Nu * (double)c->g.Nu;
+    L.scale = c->g.scale;
+    L.az_max = L.scale * (0.5 * c->g.Nz + std::fabs((double)c->g.cz) + 64.);   // with z padding
     L.accumulate = accumulate;
     return tkv::launch_backproject(store_dtype, L, st);
 }

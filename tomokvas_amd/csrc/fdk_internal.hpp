@@ -108,6 +108,7 @@ struct BPLaunch {
     int Nu, Nv, nang, pitch;
     int Nx, Ny, Nz;
     double cX, cZ, D, out_scale, maskR2;
+    double scale, az_max;   // voxel pitch, largest |z| of a z-run
     int accumulate;
 };
 int launch_backproject(int store_dtype, const BPLaunch &a, hipStream_t st);
