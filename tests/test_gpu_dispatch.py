@@ -120,6 +120,18 @@ BP_CASES = {
     "coarse": dict(Nu=90, Nv=100, Nang=9, Nx=40, Ny=37, Nz=40, D=500.0, scale=2.3),
     "near": dict(Nu=64, Nv=64, Nang=70, Nx=50, Ny=50, Nz=50, D=54.0, scale=1.1),
     "tall": dict(Nu=64, Nv=24, Nang=130, Nx=48, Ny=48, Nz=99, D=200.0, scale=1.25, cX=29.5),
+    # blocks of 16^3 voxels either side of each change of shape (128, 256, 1024,
+    # 8192), with fewer angles than groups, and with more than one batch of 64
+    "one": dict(Nu=24, Nv=20, Nang=1, Nx=9, Ny=7, Nz=5, D=90.0, scale=1.5),
+    "128": dict(Nu=130, Nv=60, Nang=66, Nx=128, Ny=127, Nz=30, D=400.0),
+    "136": dict(Nu=130, Nv=60, Nang=3, Nx=129, Ny=70, Nz=42, D=400.0),
+    "256": dict(Nu=200, Nv=40, Nang=70, Nx=250, Ny=256, Nz=16, D=500.0, scale=0.8),
+    "272": dict(Nu=260, Nv=40, Nang=5, Nx=257, Ny=250, Nz=15, D=700.0),
+    "1024": dict(Nu=260, Nv=20, Nang=67, Nx=511, Ny=512, Nz=15, D=900.0, scale=0.5),
+    "1056": dict(Nu=260, Nv=20, Nang=4, Nx=513, Ny=505, Nz=14, D=900.0, scale=0.5),
+    "8192": dict(Nu=1100, Nv=40, Nang=5, Nx=1024, Ny=1020, Nz=20, D=2000.0),
+    "8320": dict(Nu=1100, Nv=40, Nang=5, Nx=1025, Ny=1010, Nz=20, D=2000.0),
+    "8450": dict(Nu=2300, Nv=70, Nang=3, Nx=1040, Ny=1040, Nz=17, D=3800.0, scale=2.2),
 }
 
 

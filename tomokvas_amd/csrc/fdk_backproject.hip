@@ -9,7 +9,9 @@
 // MI355X design:
 //  * a workgroup owns a block of 16x16 columns x ZR slices; a thread owns one
 //    (x,y) column and its ZR slices in registers: S, T, U, u = T*U + cX and U^2
-//    depend only on (x, y, beta) and are paid once per ZR updates;
+//    depend only on (x, y, beta) and are paid once per ZR updates.  Smaller
+//    volumes take shorter runs, and G groups of threads that share a block's
+//    angles (bp_shape);
 //  * per angle, the block's detector footprint -- a box of samples that the
 //    workgroup derives from its corner columns (u and U are linear-fractional
 //    in (aX, aY), so their extremes over the block sit at the corners) -- is
@@ -312,7 +314,7 @@ struct BoxStage {
     Raw raw[PER];
 
     __device__ __forceinline__ void issue(const char *proj, int bu0, int bv0, int bh,
-                                          uint32_t row_bytes, int Nv)
+                                          uint32_t row_bytes, int Nv, int tid)
     {
         // buffer loads: a scalar descriptor at the box origin whose range ends
         // with the last row inside the detector, so rows past it read as zero
@@ -323,7 +325,7 @@ struct BoxStage {
         const int nrec = (rows + 1) * (int)row_bytes - bu0 * ST::BYTES;
         const __amdgpu_buffer_rsrc_t rsrc =
             __builtin_amdgcn_make_buffer_rsrc((void *)base, (short)0, nrec, 0x00020000);
-        int off = (int)((threadIdx.x >> 4) * row_bytes + (threadIdx.x & 15) * 4 * ST::BYTES);
+        int off = (int)((uint32_t)(tid >> 4) * row_bytes + (tid & 15) * 4 * ST::BYTES);
         // the packed-FP16 kernel forms the PER offsets anew for every box: held,
         // they would take it past the 96 registers of five waves per SIMD
         if constexpr (ST::PAIRS) asm volatile("" : "+v"(off));
@@ -344,9 +346,9 @@ struct BoxStage {
     // inside the box (bh uniform: a scalar branch); rows past the box in the
     // last block were loaded as zeros (outside the descriptor range), so the
     // tile stays finite
-    __device__ __forceinline__ void commit(float *box, int bh) const
+    __device__ __forceinline__ void commit(float *box, int bh, int tid) const
     {
-        const int r0 = threadIdx.x >> 4, col = (threadIdx.x & 15) * 4;
+        const int r0 = tid >> 4, col = (tid & 15) * 4;
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
             if (16 * i > bh) break;
@@ -395,8 +397,10 @@ __device__ __forceinline__ float div_normal(float n, float d)
 }
 
 // ---- the backprojector --------------------------------------------------------------
-template <typename S, int ZR, int LB>
-__global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
+// G: 256-thread groups of a workgroup, each with its own box, that take the
+// staged angles in turn; their sums meet in LDS at the end (see bp_shape)
+template <typename S, int ZR, int LB, int G>
+__global__ void __launch_bounds__(256 * G) bp_kernel(BPArgs<typename Store<S>::R> a)
 {
     using R = typename Store<S>::R;
     using ST = Store<S>;
@@ -405,15 +409,16 @@ __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
     constexpr int P = ST::P;
     constexpr int INNER_U = 1 << 30;   // flag beside an angle's index
     static_assert(P >= BOX_W && P % 4 == 0, "box pitch");
-    extern __shared__ __align__(16) float boxmem[];   // a.box_h rows of P words
-    // per group of 64 angles, in two slots (groups g and g+1): the staged angles,
-    // inner ones first (first column and last row of the footprint, its first
-    // row, the angle's index, cos), with their sin and scale; the number of inner
-    // and of all staged angles; and whether any angle is left to pass 2.  (Kept
-    // within 3 KiB, so that five FP16 workgroups fit a CU.)
+    extern __shared__ __align__(16) float bp_mem[];   // per group a.box_h rows of P words
+    // per batch of 64 angles, in two slots (batches g and g+1): each group's
+    // staged angles, inner ones first (first column and last row of the footprint,
+    // its first row, the angle's index, cos), with their sin and scale; the
+    // numbers of inner and of all staged angles of each group; and whether any
+    // angle is left to pass 2.  (Kept within 3 KiB, so that five FP16 workgroups
+    // fit a CU.)
     __shared__ int4 ebox[STAGED ? 128 : 1];
     __shared__ float2 ess[STAGED ? 128 : 1];
-    __shared__ int counts[4];
+    __shared__ int2 counts[2 * G];
     __shared__ int hbm_flag;
 
     // XCD-aware block order: hardware dispatches workgroup i to XCD i % 8; the
@@ -429,7 +434,10 @@ __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
     const int tile = lb - zr * a.tiles_xy;
     const int ty = tile / a.tiles_x, tx = tile - ty * a.tiles_x;
 
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int grp = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    const int tid = G == 1 ? threadIdx.x : threadIdx.x & 255;   // within the group
+    float *boxmem = bp_mem + grp * (P * a.box_h);
+    const int lane = threadIdx.x & 63, wave = tid >> 6;
     const int x = tx * 16 + (wave & 1) * 8 + (lane & 7);
     const int y = ty * 16 + (wave >> 1) * 8 + (lane >> 3);
     const int z0 = zr * ZR;
@@ -474,7 +482,7 @@ __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
         const float cy0 = (float)a.ay[ya], cy1 = (float)a.ay[yb];
 
         // pass 1: angles whose footprint fits the LDS tile.  Wave 0 evaluates
-        // a group's 64 footprints (one per lane) and sorts the staged angles
+        // a batch's 64 footprints (one per lane) and sorts the staged angles
         // into inner ones (every tap row inside the detector: gathers without
         // range tests) and edge ones; each kind runs in a loop of its own, so
         // the accumulators never pass a branch merge (which costs a copy of
@@ -486,7 +494,7 @@ __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
         if constexpr (STAGED) {
             const bool any_in = __any(inside), all_in = __all(inside);
             auto angles_of_group = [&](int g) {
-                if (wave != 0) return;
+                if (threadIdx.x >= 64) return;
                 const int bb = g * 64 + lane, slot = g & 1;
                 int4 q = make_int4(0, 0, 0, 0);
                 float c = 0.f, s = 0.f;
@@ -496,10 +504,13 @@ __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
                     q = footprint(c, s, cx0, cx1, cy0, cy1, azlo, azhi, a.cX, a.cZ, a.D, a.Nu,
                                   a.Nv, a.box_h);
                 }
+                // this lane's angle belongs to group lane % G; its rank among the
+                // lanes below of the group and kind, inner ones first
                 const bool staged = q.z > 0, inner = staged && (q.z & BOX_INNER_V);
-                const uint64_t mi = __ballot(inner), me = __ballot(staged && !inner);
+                const uint64_t own = (G == 4 ? 0x1111111111111111ull
+                                      : G == 2 ? 0x5555555555555555ull : ~0ull) << (lane % G);
+                const uint64_t mi = __ballot(inner) & own, me = __ballot(staged && !inner) & own;
                 const uint64_t mh = __ballot(q.z < 0);
-                // rank among the lanes below of the same kind, inner ones first
                 const uint64_t mk = inner ? mi : me;
                 const int rank =
                     __builtin_amdgcn_mbcnt_hi((unsigned)(mk >> 32),
@@ -508,21 +519,19 @@ __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
                 if (staged) {
                     // the index with a flag: every tap column lies on the detector
                     // (columns are below 8192, a box has at most 127 rows)
-                    ebox[slot * 64 + rank] =
-                        make_int4(q.x | q.w << 16, q.y, bb | (q.z & BOX_INNER_U ? INNER_U : 0),
-                                  __float_as_int(c));
-                    ess[slot * 64 + rank] = make_float2(s, a.scales[bb] * wnorm);
+                    const int at = slot * 64 + (lane % G) * (64 / G) + rank;
+                    ebox[at] = make_int4(q.x | q.w << 16, q.y,
+                                         bb | (q.z & BOX_INNER_U ? INNER_U : 0), __float_as_int(c));
+                    ess[at] = make_float2(s, a.scales[bb] * wnorm);
                 }
-                if (lane == 0) {
-                    counts[2 * slot] = __popcll(mi);
-                    counts[2 * slot + 1] = __popcll(mi) + __popcll(me);
-                    if (mh) hbm_flag = 1;
-                }
+                if (lane < G)
+                    counts[slot * G + lane] = make_int2(__popcll(mi), __popcll(mi) + __popcll(me));
+                if (lane == 0 && mh) hbm_flag = 1;
             };
             auto uniform_int = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
             // the tile starts finite: rows of a box past its last 16-row block
             // are never written
-            for (int i = threadIdx.x; i < P * a.box_h; i += 256) boxmem[i] = 0.f;
+            for (int i = tid; i < P * a.box_h; i += 256) boxmem[i] = 0.f;
             if (threadIdx.x == 0) hbm_flag = 0;
             __syncthreads();
             angles_of_group(0);
@@ -538,7 +547,7 @@ __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
                 bv0 = uniform_int(e.y);
                 bi = uniform_int(e.z);
                 stage.issue(a.stack + (size_t)(bi & ~INNER_U) * a.angle_bytes, bu0, bv0, bh,
-                            a.row_bytes, a.Nv);
+                            a.row_bytes, a.Nv, tid);
             };
             // column weights and LDS offsets of the staged angle, then its gathers
             auto gather_angle = [&](auto fast_tag, int qu, int qv, bool inner_u, float wc, float ws,
@@ -586,42 +595,56 @@ __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
             for (int g = 0; g < ngroups; ++g) {
                 const int slot = g & 1;
                 if (g > 0) {
-                    // the slot of group g-1 is free once every wave is here
+                    // the slot of batch g-1 is free once every wave is here
                     __syncthreads();
                     angles_of_group(g + 1);
                     __syncthreads();
                 }
-                const int ni = uniform_int(counts[2 * slot]), n = uniform_int(counts[2 * slot + 1]);
-                const int n1 = uniform_int(counts[2 * (slot ^ 1) + 1]);
-                if (!loading && n > 0) issue(ebox[slot * 64]);
-                loading = n > 0 && g + 1 < ngroups && n1 > 0;
-                // entries [e0, e1); while one is gathered the next one's box is
-                // loaded (the next group's first after the last)
-                auto run = [&](auto fast_tag, int e0, int e1) {
-                    for (int j = e0; j < e1; ++j) {
+                // this group's inner and staged angles, the most of any group, and
+                // whether this group has any in the next batch
+                const int ni = uniform_int(counts[slot * G + grp].x);
+                const int n = uniform_int(counts[slot * G + grp].y);
+                int mi = ni, me = n - ni;
+                for (int h = 0; h < G; ++h) {
+                    const int hi = uniform_int(counts[slot * G + h].x);
+                    mi = max(mi, hi);
+                    me = max(me, uniform_int(counts[slot * G + h].y) - hi);
+                }
+                const bool next = g + 1 < ngroups && uniform_int(counts[(slot ^ 1) * G + grp].y) > 0;
+                const int base = slot * 64 + grp * (64 / G), base1 = base ^ 64;
+                if (!loading && n > 0) issue(ebox[base]);
+                loading = n > 0 && next;
+                // t-th of this group's entries [e0, e1), `most` steps; while one is
+                // gathered the next one's box is loaded (the next batch's first
+                // after the last)
+                auto run = [&](auto fast_tag, int e0, int e1, int most) {
+                    for (int t = 0; t < most; ++t) {
+                        const int j = e0 + t;
+                        const bool mine = G == 1 || j < e1;
                         const int qu = bu0, qv = bv0, qh = bh;
                         const bool inner_u = bi & INNER_U;
-                        const int at = j + 1 < n ? slot * 64 + j + 1 : (slot ^ 1) * 64;
-                        const bool more = j + 1 < n || loading;
-                        const int4 e = ebox[at];            // (read, not used, if no more)
-                        const float wc = __int_as_float(ebox[slot * 64 + j].w);
-                        const float2 ss = ess[slot * 64 + j];
+                        const bool more = mine && (j + 1 < n || loading);
+                        const int4 e = ebox[j + 1 < n ? base + j + 1 : base1];
+                        const int at = base + (mine ? j : 0);
+                        const float wc = __int_as_float(ebox[at].w);
+                        const float2 ss = ess[at];
                         __syncthreads();   // every wave is done with the previous box
-                        stage.commit(boxmem, qh);
+                        if (mine) stage.commit(boxmem, qh, tid);
                         __syncthreads();
                         if (more) issue(e);
-                        if (any_in) gather_angle(fast_tag, qu, qv, inner_u, wc, ss.x, ss.y);
+                        if (mine && any_in)
+                            gather_angle(fast_tag, qu, qv, inner_u, wc, ss.x, ss.y);
                     }
                 };
-                run(fast_t{}, 0, ni);
-                run(edge_t{}, ni, n);
+                run(fast_t{}, 0, ni, mi);
+                run(edge_t{}, ni, n, me);
             }
             need_hbm = uniform_int(hbm_flag) != 0;
         }
 
         // pass 2: angles gathered straight from HBM -- all of them for FP64,
         // and those whose box exceeds the LDS tile for the staged types
-        if (need_hbm && __any(inside)) {
+        if (need_hbm && grp == 0 && __any(inside)) {
             const char *proj = a.stack;
             for (int b = 0; b < a.nang; ++b, proj += a.angle_bytes) {
                 if constexpr (STAGED) {
@@ -662,6 +685,30 @@ __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
         }
     }
 
+    if constexpr (G > 1) {
+        // the groups' sums, through LDS in pieces that fit one box (at least 16
+        // rows), added in the order of the groups
+        constexpr int BP_PIECE = 4;
+        static_assert(BP_PIECE * 256 <= 16 * P, "piece of the group sums beyond a box");
+#pragma unroll
+        for (int h = 1; h < G; ++h)
+#pragma unroll
+            for (int k0 = 0; k0 < ZR; k0 += BP_PIECE) {
+                __syncthreads();
+                if (grp == h) {
+#pragma unroll
+                    for (int k = 0; k < BP_PIECE; ++k)
+                        if (k0 + k < ZR) bp_mem[k * 256 + tid] = acc[k0 + k];
+                }
+                __syncthreads();
+                if (grp == 0) {
+#pragma unroll
+                    for (int k = 0; k < BP_PIECE; ++k)
+                        if (k0 + k < ZR) acc[k0 + k] += bp_mem[k * 256 + tid];
+                }
+            }
+        if (grp > 0) return;
+    }
     if (!valid_xy) return;
     const size_t plane = (size_t)a.Nx * a.Ny;
     R *out = a.vol + (size_t)y * a.Nx + x;
@@ -678,7 +725,7 @@ __global__ void __launch_bounds__(256) bp_kernel(BPArgs<typename Store<S>::R> a)
     }
 }
 
-int bp_zrun(int dtype)
+static int native_zrun(int dtype)
 {
     switch (dtype) {
     case FDK_F32: return Store<st_f32>::ZR;
@@ -688,6 +735,37 @@ int bp_zrun(int dtype)
     case FDK_F64: return Store<st_f64>::ZR;
     default: return 0;
     }
+}
+
+// The long z-runs (slices per thread, TKV_BP_ZR_*) spread a column's set-up over the most updates and read each
+// box row for the most slices, but a volume of few blocks leaves CUs idle, or ends
+// on a mostly idle last wave.  So a smaller volume takes runs of 16 slices, and one
+// whose blocks still don't fill the 256 CUs has 2 or 4 groups of 256 threads per
+// block, each gathering every 2nd or 4th angle from a box of its own; their sums
+// meet in LDS.  By blocks of 16^3 voxels; us for 32-slice (FP32: 24) runs, runs of
+// 16 with 1, 2, 4 groups, runs of 8 with 4 groups:
+//      8  32^3, 36 angles              60    45    33    30    22
+//     64  64^3, 90 angles             142   100    72    61    44
+//    108  96^2 x 40, 120, FP16        232   145    98    79    54
+//    180  96^2 x 80, 150, BF16        292   159   114    94   129
+//    512  128^3, 180                  320   224   186   218   284
+//   1000  160^2 x 150, 240, BF16      557   441   446   567   731
+//   1690  203^2 x 157, 251            741   689   792   951  1313
+//   4096  256^3, 360                 2026  1939  2410  3003  4013
+//   7600  320^2 x 300, 360, BF16     3519  3221  3594  5539  7860
+//  15625  400^3, 400                 7403  7543  9556 12319 17095
+// Taken from the whole volume and from neither the angles nor the slices of one
+// launch, so that a volume in z-chunks gets the sums of one launch.  (FP64 gathers
+// from HBM without boxes and keeps its runs of 8.)
+BPShape bp_shape(int dtype, int Nx, int Ny, int Nz)
+{
+    const int native = native_zrun(dtype);
+    const long long n = (long long)((Nx + 15) / 16) * ((Ny + 15) / 16) * ((Nz + 15) / 16);
+    if (dtype == FDK_F64 || n > 8192) return {native, 1, native};
+    if (n <= 128) return {8, 4, 32};
+    if (n <= 256) return {16, 4, 32};
+    if (n <= 1024) return {16, 2, 32};
+    return {16, 1, 32};
 }
 
 int sample_bytes_of(int dtype)
@@ -719,11 +797,10 @@ static int box_height(const BPLaunch &L)
     return rows >= most ? most : ((int)rows + 16) / 16 * 16;
 }
 
-template <typename S>
-static int launch_bp_t(const BPLaunch &L, hipStream_t st)
+template <typename S, int ZR, int G>
+static int launch_bp_z(const BPLaunch &L, hipStream_t st)
 {
     using R = typename Store<S>::R;
-    constexpr int ZR = Store<S>::ZR;
     if (L.pitch < stack_pitch(L.Nu))
         return fail(FDK_ERR_INVALID_ARGUMENT, "backproject: stack pitch below the padded width");
     BPArgs<R> a;
@@ -760,10 +837,30 @@ static int launch_bp_t(const BPLaunch &L, hipStream_t st)
     if (!grid_fits(nb, 256)) return fail(FDK_ERR_UNSUPPORTED, "backproject: volume too large");
     a.nblocks = (int)nb;
     a.box_h = Store<S>::STAGED ? box_height<ZR>(L) : 0;
-    hipLaunchKernelGGL((bp_kernel<S, ZR, (ZR < TKV_BP_LB ? ZR : TKV_BP_LB)>), dim3((unsigned)nb),
-                       dim3(256), sizeof(float) * Store<S>::P * a.box_h, st, a);
+    constexpr int LB = ZR < TKV_BP_LB ? ZR : TKV_BP_LB;
+    const size_t lds = sizeof(float) * Store<S>::P * a.box_h * G;
+    // beyond 64 KiB a workgroup takes up to the 160 KiB of LDS of a gfx950 CU
+    if (lds > 61440)
+        TKV_HIP(hipFuncSetAttribute((const void *)bp_kernel<S, ZR, LB, G>,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL((bp_kernel<S, ZR, LB, G>), dim3((unsigned)nb), dim3(256 * G), lds, st, a);
     TKV_HIP(hipGetLastError());
     return FDK_OK;
+}
+
+template <typename S>
+static int launch_bp_t(const BPLaunch &L, hipStream_t st)
+{
+    constexpr int ZR = Store<S>::ZR;
+    const int z = L.shape.zrun, g = L.shape.groups;
+    if (z == ZR && g == 1) return launch_bp_z<S, ZR, 1>(L, st);
+    if constexpr (Store<S>::STAGED) {
+        if (z == 8 && g == 4) return launch_bp_z<S, 8, 4>(L, st);
+        if (z == 16 && g == 4) return launch_bp_z<S, 16, 4>(L, st);
+        if (z == 16 && g == 2) return launch_bp_z<S, 16, 2>(L, st);
+        if (z == 16 && g == 1) return launch_bp_z<S, 16, 1>(L, st);
+    }
+    return fail(FDK_ERR_INVALID_ARGUMENT, "backproject: no kernel of this shape");
 }
 
 int launch_backproject(int dtype, const BPLaunch &a, hipStream_t st)

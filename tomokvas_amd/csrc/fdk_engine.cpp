@@ -356,6 +356,8 @@ int stage_backproject(fdk_ctx *c, int store_dtype, const void *stack, const void
     L.scale = c->g.scale;
     L.az_max = L.scale * (0.5 * c->g.Nz + std::fabs((double)c->g.cz) + 64.);   // with z padding
     L.accumulate = accumulate;
+    // from the whole volume, so that a volume in z-chunks gets the same sums
+    L.shape = tkv::bp_shape(store_dtype, c->g.Nx, c->g.Ny, c->g.Nz);
     return tkv::launch_backproject(store_dtype, L, st);
 }
 
@@ -474,7 +476,7 @@ int backproject_in_angle_chunks(fdk_ctx *c, const std::vector<int> &ab, void *vo
 int pipeline_chunk(const fdk_ctx *c)
 {
     const tkv::Geometry &g = c->g;
-    const int zr = tkv::bp_zrun(c->storage);
+    const int zr = tkv::bp_shape(c->storage, g.Nx, g.Ny, g.Nz).chunk;
     if (c->volume_mode != FDK_VOLUME_STREAMED) return chunk_target(g, zr, TKV_HANDOUT_ZPARTS);
     int C = chunk_target(g, zr, 8);
     if (c->ring_slices < g.Nz) C = std::min(C, (c->ring_slices - g.B) / 2 / zr * zr);
@@ -511,7 +513,7 @@ int backproject_and_hand_out(fdk_ctx *c, fdk_get_block_fn get_block, void *user,
     float *ring = streamed ? c->d_ring : c->d_vol;
     const bool wraps = W < g.Nz;
     const int C = pipeline_chunk(c);
-    const int zr = tkv::bp_zrun(c->storage);
+    const int zr = tkv::bp_shape(c->storage, g.Nx, g.Ny, g.Nz).chunk;
     if (C < 1 || (wraps && 2 * C + g.B > W))
         return fail(FDK_ERR_INVALID_ARGUMENT, "slab pipeline: volume buffer too small");
     // a ring slot holds other slices before its chunk is backprojected: only a

@@ -99,6 +99,13 @@ int launch_accumulate(float *dst, const float *src, size_t n, hipStream_t st);
 int launch_zero_u32(unsigned *dst, size_t n, hipStream_t st);
 int launch_compare(const float *a, const float *b, size_t n, double *d_out3, hipStream_t st);
 
+// How the backprojector cuts a volume: slices per thread, 256-thread groups that
+// share a block's angles, and the multiple of slices at which a volume may be cut
+// into launches without cutting a z-run.
+struct BPShape {
+    int zrun, groups, chunk;
+};
+
 struct BPLaunch {
     const void *stack;      // [nang][Nv][pitch] in the storage type
     const void *scales;     // per local angle dequantisation factor (Real)
@@ -110,9 +117,10 @@ struct BPLaunch {
     double cX, cZ, D, out_scale, maskR2;
     double scale, az_max;   // voxel pitch, largest |z| of a z-run
     int accumulate;
+    BPShape shape;
 };
 int launch_backproject(int store_dtype, const BPLaunch &a, hipStream_t st);
-int bp_zrun(int store_dtype);
+BPShape bp_shape(int store_dtype, int Nx, int Ny, int Nz);
 int sample_bytes_of(int store_dtype);   // bytes of one stored sample
 int stack_pitch(int Nu);                // row pitch of the stored stack, samples
 constexpr int STACK_TAIL_ROWS = 128;    // spare rows after the last projection (>= box rows)
