@@ -1,6 +1,7 @@
 """Kernels and dispatch rules at the sizes where they can go wrong, each
 against the oracle or the general path."""
 import ctypes as C
+import math
 import threading
 
 import numpy as np
@@ -155,3 +156,61 @@ def test_backprojection_boxes(torch, case, store):
     dec = (q * scales[:, None, None]).transpose(0, 1).contiguous()
     ref = O.backproject(ogeom(g), dec.cpu().numpy())
     assert O.rel_rmse(got, ref) <= 1e-6
+
+
+# (sin_x, sin_y, n, axis): one column, one row, an odd sinogram left over, one to
+# several waves side by side, rows that end inside a wave's
+RSQ_SIZES = [(1, 1, 1, 0), (2, 3, 3, 0), (64, 37, 2, 0), (65, 361, 5, 1), (130, 100, 3, 2),
+             (300, 203, 1, 40), (513, 90, 4, 0)]
+
+
+@pytest.mark.parametrize("size", RSQ_SIZES)
+@pytest.mark.parametrize("step", [1.0, 0.93, 1.21])
+def test_rsq_full_fan(torch, size, step):
+    """The one-pass rebinning against the reference's formula over whole rows, for
+    angle steps of a full turn and others (whose pairs wrap around the scan), with
+    columns without flat field and counts at and below dark."""
+    from oracle import rsq as R
+    from rsq_util import synthetic_raw
+
+    sx, sy, n, axis = size
+    raw = synthetic_raw(n, sy, sx, seed=sx)
+    raw[:, 1, ::29] = raw[:, 0, ::29]                # flat = dark
+    raw[:, 1, 7::31] = 50                            # flat < dark
+    raw[:, 2::11, 3::13] = raw[:, :1, 3::13]         # count = dark
+    raw[:, 5::17, 1::19] = 3                         # count < dark
+    L = _lib.load()
+    p = _lib.RsqParams()
+    _lib.check(L.fdk_rsq_default_params(C.byref(p)), "rsq params")
+    p.sin_x, p.sin_y, p.axis_move, p.complete, p.flip = sx, sy, axis, 1, sx % 2
+    p.distance, p.delta_fi = 4.0 * sx, step * 2 * math.pi / sy
+    w = 2 * sx - 1 - 2 * axis
+    d_raw = torch.from_numpy(raw.view(np.int16)).cuda()
+    got = {}
+    for dt, store in ((torch.float64, _lib.F64), (torch.float32, _lib.F32)):
+        out = torch.zeros((n, sy, w), device="cuda", dtype=dt)
+        say(f"rsq {size} step {step} dtype {store}")
+        _lib.check(L.fdk_rsq_process(C.byref(p), 1.1, 0.1, C.c_void_p(d_raw.data_ptr()), n, store,
+                                     C.c_void_p(out.data_ptr()), None), "rsq")
+        got[store] = out.cpu().numpy()
+    f = np.arange(sy)[:, None]
+    c0 = sx - 1 - axis
+    t = np.arange(-c0, 0)
+    base = f * p.delta_fi - 2 * np.arctan(t / p.distance)
+    nf = (base - math.pi) / p.delta_fi
+    nf = np.where((nf > sy - 1) | (nf < 0), (base + math.pi) / p.delta_fi, nf)
+    ca, fl = np.ceil(nf), np.floor(nf)
+    want = np.empty((n, sy, w))
+    with np.errstate(invalid="ignore"):
+        for k in range(n):
+            ff = R.flat_field(raw[k], 1.1, 0.1, False)
+            A, B = (ff[(v.astype(np.int64) % sy), axis - t] for v in (ca, fl))
+            want[k, :, :c0] = np.where(ca != fl, A + (B - A) * (ca - nf), A)
+            want[k, :, c0:] = ff[:, axis:]
+    if p.flip:
+        want = want[:, ::-1]
+    fin = np.isfinite(want)
+    assert np.array_equal(got[_lib.F64][~fin], want[~fin], equal_nan=True)
+    err = np.abs(got[_lib.F64] - want)[fin]
+    assert err.size == 0 or err.max() <= 1e-12 * max(np.abs(want[fin]).max(), 1.0)
+    np.testing.assert_array_equal(got[_lib.F32], got[_lib.F64].astype(np.float32))
