@@ -214,3 +214,38 @@ def test_rsq_full_fan(torch, size, step):
     err = np.abs(got[_lib.F64] - want)[fin]
     assert err.size == 0 or err.max() <= 1e-12 * max(np.abs(want[fin]).max(), 1.0)
     np.testing.assert_array_equal(got[_lib.F32], got[_lib.F64].astype(np.float32))
+
+
+def test_prepare_again_equals_a_new_context(torch):
+    """One context prepared for one geometry and filter after another -- larger
+    tables, smaller ones, other taps -- filters and backprojects as a context
+    prepared once does."""
+    from tomokvas_amd import diff
+    from tomokvas_amd.stages import Stages
+
+    sizes = [dict(Nu=40, Nv=12, Nang=9, Nx=24, Ny=20, Nz=16, D=200.0),
+             dict(Nu=140, Nv=30, Nang=37, Nx=50, Ny=48, Nz=90, D=500.0),
+             dict(Nu=40, Nv=12, Nang=9, Nx=24, Ny=20, Nz=16, D=300.0)]
+    one = None
+    for i, kw in enumerate(sizes):
+        g = scan(**kw)
+        fresh = stages(g)
+        if one is None:
+            one = stages(g)
+        else:
+            fbp = one.fbp
+            g.apply(fbp, None, None)
+            _lib.check(fbp.SetFilter(_lib.FILTER_RAMLAK), "SetFilter")
+            one = Stages(fbp)
+        for taps in (None, np.random.default_rng(i).standard_normal(fresh.p)):
+            say(f"prepare again {i} taps {taps is not None}")
+            got = []
+            for st in (fresh, one):
+                if taps is not None:
+                    diff.set_taps(st, taps)
+                gen = torch.Generator(device="cuda").manual_seed(i)
+                d = torch.randn(st.sino_shape(), device="cuda", generator=gen)
+                st.filter(d, weight=True)
+                stack, scales = st.pack(d, _lib.F32)
+                got.append(st.backproject(stack, _lib.F32, scales).cpu())
+            assert torch.equal(got[0], got[1])

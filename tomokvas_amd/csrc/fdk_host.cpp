@@ -127,47 +127,18 @@ static double shepplogan(int n, double tau)
     return -2. / (M_PI * M_PI * tau * tau * (4. * (double)n * (double)n - 1.));
 }
 
-// DFT_p of real x for bins [0, kmax), twiddle index reduced mod p.
-static void dft(const std::vector<double> &x, int p, int kmax, std::vector<double> &re,
-                std::vector<double> &im)
-{
-    std::vector<double> c(p), s(p);
-    for (int j = 0; j < p; ++j) {
-        double a = 2.0 * M_PI * (double)j / (double)p;
-        c[j] = std::cos(a);
-        s[j] = std::sin(a);
-    }
-    std::vector<int> nz;
-    for (int n = 0; n < p; ++n)
-        if (x[n] != 0.) nz.push_back(n);
-    re.assign(kmax, 0.);
-    im.assign(kmax, 0.);
-    for (int k = 0; k < kmax; ++k) {
-        double sr = 0., si = 0.;
-        for (int n : nz) {
-            int j = (int)(((long long)k * n) % p);
-            sr += x[n] * c[j];
-            si -= x[n] * s[j];
-        }
-        re[k] = sr;
-        im[k] = si;
-    }
-}
-
 // FillFilter + R2C + AbsKernel (kernel.cu:585, 620-646, 783-790): taps
 // t[i] = h(i - Nu/2)/2 for i < Nu, zero-padded to p; spectrum tau*|DFT(t)|,
 // evenly extended to the full length p (Hermitian symmetry of the R2C output).
 void build_spectrum(int kind, const Geometry &g, const std::vector<double> &user_taps,
-                    std::vector<double> &Hre, std::vector<double> &Him)
+                    const std::vector<double> &tw, std::vector<double> &Hre,
+                    std::vector<double> &Him)
 {
     const int p = padded_length(g.Nu);
-    Hre.assign(p, 0.);
     Him.assign(p, 0.);
     if (kind == FDK_FILTER_USER) {
-        std::vector<double> re, im;
-        dft(user_taps, p, p, re, im);
-        Hre = re;
-        Him = im;
+        Hre = user_taps;
+        fft_pow2(Hre, Him, tw);
         return;
     }
     const double tau = (double)g.tau;
@@ -176,16 +147,17 @@ void build_spectrum(int kind, const Geometry &g, const std::vector<double> &user
         int n = i - g.Nu / 2;
         t[i] = (kind == FDK_FILTER_SHEPPLOGAN ? shepplogan(n, tau) : ramlak(n, tau)) / 2.;
     }
-    std::vector<double> re, im;
-    dft(t, p, p / 2 + 1, re, im);
+    std::vector<double> im(p, 0.);
+    fft_pow2(t, im, tw);
+    Hre.assign(p, 0.);
     for (int k = 0; k <= p / 2; ++k) {
-        double a = tau * std::sqrt(re[k] * re[k] + im[k] * im[k]);
+        double a = tau * std::sqrt(t[k] * t[k] + im[k] * im[k]);
         Hre[k] = a;
         if (k > 0 && k < p / 2) Hre[p - k] = a;
     }
 }
 
-void fft_pow2(std::vector<double> &re, std::vector<double> &im)
+void fft_pow2(std::vector<double> &re, std::vector<double> &im, const std::vector<double> &tw)
 {
     const size_t n = re.size();
     // bit-reversal permutation
@@ -199,12 +171,10 @@ void fft_pow2(std::vector<double> &re, std::vector<double> &im)
         }
     }
     for (size_t len = 2; len <= n; len <<= 1) {
-        const size_t half = len >> 1;
-        for (size_t k = 0; k < half; ++k) {
-            // e^{-2 pi i k / len}
-            const double a = -2.0 * M_PI * (double)k / (double)len;
-            const double wr = std::cos(a), wi = std::sin(a);
-            for (size_t s0 = 0; s0 < n; s0 += len) {
+        const size_t half = len >> 1, step = n / len;
+        for (size_t s0 = 0; s0 < n; s0 += len) {
+            for (size_t k = 0; k < half; ++k) {
+                const double wr = tw[2 * k * step], wi = tw[2 * k * step + 1];
                 const size_t i0 = s0 + k, i1 = i0 + half;
                 const double xr = re[i1] * wr - im[i1] * wi;
                 const double xi = re[i1] * wi + im[i1] * wr;

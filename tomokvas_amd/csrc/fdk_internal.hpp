@@ -62,11 +62,14 @@ int slab_count(int Nz, int B);
 // filter spectrum in FP64 (kernel.cu:570-655, 783-802):
 //   kind RAMLAK / SHEPPLOGAN: H[k] = tau*|DFT_p(t)[k]| real, k in [0,p)
 //   kind USER: H[k] = DFT_p(h)[k] complex for the caller's p spatial taps
+//   (tw: the p twiddles as fft_pow2 takes them)
 void build_spectrum(int kind, const Geometry &g, const std::vector<double> &user_taps,
-                    std::vector<double> &Hre, std::vector<double> &Him);
+                    const std::vector<double> &tw, std::vector<double> &Hre,
+                    std::vector<double> &Him);
 // in-place forward DFT X[j] = sum_k x[k] e^{-2 pi i k j / n} in double, n a
-// power of two (iterative radix-2; twiddles from the exact index)
-void fft_pow2(std::vector<double> &re, std::vector<double> &im);
+// power of two (iterative radix-2; tw: e^{-2 pi i j / n} as (re, im) pairs, each
+// from the exact index)
+void fft_pow2(std::vector<double> &re, std::vector<double> &im, const std::vector<double> &tw);
 
 // ---------------------------------------------------------------- kernel launchers
 // A dispatch holds its size in work-items in a 32-bit field per dimension, so a
