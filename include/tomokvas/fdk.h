@@ -192,6 +192,10 @@ int fdk_forward_project(fdk_ctx *ctx, int dtype, const void *d_vol, int ang0, in
  * q, G [Nv][nang][Nu]; accumulated into the host array dh[p] (double). */
 int fdk_tap_gradient(fdk_ctx *ctx, int dtype, const void *d_q, const void *d_G, int nang,
                      double *dh, void *stream);
+/* fdk_tap_gradient of q = W p for projections p [Nv][nang][Nu]: the cosine weight
+ * (fdk_weight) is applied as the rows are loaded. */
+int fdk_tap_gradient_weighted(fdk_ctx *ctx, int dtype, const void *d_p, const void *d_G,
+                              int nang, double *dh, void *stream);
 /* fdk_tap_gradient without any allocation: no counterpart in the reference; for
  * callers that cannot allocate (code under HIP graph capture, tight training
  * loops, harnesses that forbid hipMalloc).  Its partial spectra live in a

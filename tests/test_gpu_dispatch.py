@@ -249,3 +249,30 @@ def test_prepare_again_equals_a_new_context(torch):
                 stack, scales = st.pack(d, _lib.F32)
                 got.append(st.backproject(stack, _lib.F32, scales).cpu())
             assert torch.equal(got[0], got[1])
+
+
+# one row, rows that end inside a pair and a workgroup, several launches of the
+# capped grid (2048 workgroups x 4 pairs of a transform); NT = 1 to 256
+@pytest.mark.parametrize("Nu,Nv,Nang", [(1, 1, 1), (5, 3, 7), (64, 11, 29), (300, 70, 31),
+                                        (1024, 40, 601), (1500, 130, 141)])
+def test_weighted_tap_gradient(torch, Nu, Nv, Nang):
+    """The cosine weight applied as the rows are loaded gives the products of the
+    weighted rows."""
+    g = scan(Nu, Nv, Nang, 8, 8, 8, D=max(900.0, 2.0 * Nu), cX=0.4 * Nu)
+    st = stages(g)
+    gen = torch.Generator(device="cuda").manual_seed(Nu)
+    # (FP64 transforms of 4096 don't fit: refused)
+    for dt in (torch.float32, torch.float64)[:2 if st.p <= 2048 else 1]:
+        p, G = (torch.randn(st.sino_shape(), device="cuda", generator=gen, dtype=dt)
+                for _ in range(2))
+        say(f"weighted tap gradient {Nu}x{Nv}x{Nang} {dt}")
+        got = st.tap_gradient(p, G, weight=True)
+        want = st.tap_gradient(st.weight(p.clone()), G)
+        # the same products in the same order: FMA contraction of the weight into
+        # the first pass is all that may differ
+        tol = 2e-6 if dt == torch.float32 else 1e-14
+        assert np.abs(got - want).max() <= tol * max(np.abs(want).max(), 1e-30) * math.sqrt(Nu)
+        if Nu <= 64:
+            ref = O.tap_gradient(ogeom(g), st.weight(p.clone()).double().cpu().numpy(),
+                                 G.double().cpu().numpy())
+            assert np.abs(got - ref).max() <= (1e-5 if dt == torch.float32 else 1e-12) * np.abs(ref).max()

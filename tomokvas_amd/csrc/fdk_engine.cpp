@@ -1237,8 +1237,26 @@ int fdk_forward_project(fdk_ctx *c, int dtype, const void *d_vol, int ang0, int 
     return tkv::launch_forward_project(f64 ? 8 : 4, L, pick(c, stream));
 }
 
-int fdk_tap_gradient(fdk_ctx *c, int dtype, const void *d_q, const void *d_G, int nang,
-                     double *dh, void *stream)
+static tkv::TapGradLaunch tap_launch(const fdk_ctx *c, int dtype, const void *q, const void *G,
+                                     int nang, int weight)
+{
+    tkv::TapGradLaunch L;
+    L.q = q;
+    L.G = G;
+    L.Nu = c->g.Nu;
+    L.nang = nang;
+    L.rows = (long long)c->g.Nv * nang;
+    L.p = c->p;
+    L.weight = weight;
+    L.cX = c->g.cX;
+    L.cZ = c->g.cZ;
+    L.D = c->g.D;
+    L.tw = dtype == FDK_F64 ? (const void *)c->d_tw64 : (const void *)c->d_tw32;
+    return L;
+}
+
+static int tap_gradient(fdk_ctx *c, int dtype, const void *d_q, const void *d_G, int nang,
+                        int weight, double *dh, void *stream)
 {
     int rc = need_prepared(c);
     if (rc) return rc;
@@ -1249,10 +1267,10 @@ int fdk_tap_gradient(fdk_ctx *c, int dtype, const void *d_q, const void *d_G, in
     const long long rows = (long long)c->g.Nv * nang;
     const int nblocks = (int)std::max<long long>(1, std::min<long long>(tap_blocks(p, rows), 2048));
     const size_t rb = dtype == FDK_F64 ? 8 : 4;
-    // partial spectra of the workgroups, then their sum (p complex doubles)
+    // partial spectra of the workgroups, then their sums (p complex doubles each)
     const size_t pbytes = (size_t)nblocks * p * 2 * rb;
     const size_t sbytes = (size_t)p * 2 * sizeof(double);
-    const size_t bytes = pbytes + sbytes;
+    const size_t bytes = pbytes + (tkv::TAPGRAD_SPLIT + 1) * sbytes;
     if (bytes > c->scratch_bytes) {
         dfree(c->d_scratch);
         c->scratch_bytes = 0;
@@ -1260,16 +1278,11 @@ int fdk_tap_gradient(fdk_ctx *c, int dtype, const void *d_q, const void *d_G, in
         c->scratch_bytes = bytes;
     }
     hipStream_t st = pick(c, stream);
-    tkv::TapGradLaunch L;
-    L.q = d_q;
-    L.G = d_G;
-    L.Nu = c->g.Nu;
-    L.rows = (int)std::min<long long>(rows, 0x7fffffff);
-    L.p = p;
-    L.tw = dtype == FDK_F64 ? (const void *)c->d_tw64 : (const void *)c->d_tw32;
+    tkv::TapGradLaunch L = tap_launch(c, dtype, d_q, d_G, nang, weight);
     L.partial = c->d_scratch;
     L.nblocks = nblocks;
     L.spectrum = (char *)c->d_scratch + pbytes;
+    L.sums = (char *)L.spectrum + sbytes;
     if ((rc = tkv::launch_tap_gradient((int)rb, L, st))) return rc;
     std::vector<double> P(2 * (size_t)p);
     TKV_HIP(hipMemcpyAsync(P.data(), L.spectrum, sbytes, hipMemcpyDeviceToHost, st));
@@ -1285,6 +1298,18 @@ int fdk_tap_gradient(fdk_ctx *c, int dtype, const void *d_q, const void *d_G, in
     tkv::fft_pow2(Rr, Ri, c->tw);
     for (int j = 0; j < p; ++j) dh[j] += Rr[j];
     return FDK_OK;
+}
+
+int fdk_tap_gradient(fdk_ctx *c, int dtype, const void *d_q, const void *d_G, int nang,
+                     double *dh, void *stream)
+{
+    return tap_gradient(c, dtype, d_q, d_G, nang, 0, dh, stream);
+}
+
+int fdk_tap_gradient_weighted(fdk_ctx *c, int dtype, const void *d_p, const void *d_G, int nang,
+                              double *dh, void *stream)
+{
+    return tap_gradient(c, dtype, d_p, d_G, nang, 1, dh, stream);
 }
 
 // Allocation-free variant of fdk_tap_gradient for callers that cannot call
@@ -1308,9 +1333,9 @@ int fdk_tap_gradient_noalloc(fdk_ctx *c, int dtype, const void *d_q, const void 
         return fail(FDK_ERR_INVALID_ARGUMENT, "tap_gradient_noalloc: null buffer");
     const int p = c->p;
     const size_t rb = dtype == FDK_F64 ? 8 : 4;
-    // spectrum (p complex doubles) and gradient (p doubles) at the end of the
-    // scratch, the partial spectra before them
-    const size_t tail = (size_t)p * 3 * sizeof(double);
+    // spectrum, the reduction's sums (p complex doubles each) and gradient (p
+    // doubles) at the end of the scratch, the partial spectra before them
+    const size_t tail = (size_t)p * (3 + 2 * tkv::TAPGRAD_SPLIT) * sizeof(double);
     const size_t per_block = (size_t)p * 2 * rb;
     if (tail + per_block > TAPGRAD_SCRATCH)
         return fail(FDK_ERR_UNSUPPORTED,
@@ -1324,17 +1349,12 @@ int fdk_tap_gradient_noalloc(fdk_ctx *c, int dtype, const void *d_q, const void 
     char *scr = nullptr;
     if ((rc = tapgrad_scratch_of_device(c->dev, (void **)&scr))) return rc;
     hipStream_t st = pick(c, stream);
-    tkv::TapGradLaunch L;
-    L.q = d_q;
-    L.G = d_G;
-    L.Nu = c->g.Nu;
-    L.rows = (int)std::min<long long>(rows, 0x7fffffff);
-    L.p = p;
-    L.tw = dtype == FDK_F64 ? (const void *)c->d_tw64 : (const void *)c->d_tw32;
+    tkv::TapGradLaunch L = tap_launch(c, dtype, d_q, d_G, nang, 0);
     L.partial = scr;
     L.nblocks = nblocks;
     L.spectrum = scr + (TAPGRAD_SCRATCH - tail);
-    double *d_dh = (double *)((char *)L.spectrum + (size_t)p * 2 * sizeof(double));
+    L.sums = (char *)L.spectrum + (size_t)p * 2 * sizeof(double);
+    double *d_dh = (double *)((char *)L.sums + (size_t)p * 2 * tkv::TAPGRAD_SPLIT * sizeof(double));
     if ((rc = tkv::launch_tap_gradient((int)rb, L, st))) return rc;
     if ((rc = tkv::launch_tap_gradient_dft(L.spectrum, c->d_tw64, p, d_dh, st))) return rc;
     double part[512];

@@ -142,12 +142,19 @@ struct FPLaunch {           // adjoint of the backprojector
 };
 int launch_forward_project(int real_bytes, const FPLaunch &a, hipStream_t st);
 
+// row pairs of one transform whose products are summed in the data's type before
+// the sum goes on in double; sums of the reduction's first step
+constexpr int TAPGRAD_PAIRS = 4, TAPGRAD_SPLIT = 16;
 struct TapGradLaunch {
-    const void *q, *G;      // [rows][Nu] weighted input rows and output gradients
-    int Nu, rows, p;
+    const void *q, *G;      // [rows][Nu] input rows and output gradients
+    int Nu, nang, p;
+    long long rows;         // Nv * nang
+    int weight;             // q are projections: apply the cosine weight
+    float cX, cZ, D;
     const void *tw;
     void *partial;          // [nblocks][p] complex Real
     int nblocks;
+    void *sums;             // [TAPGRAD_SPLIT][p] complex double
     void *spectrum;         // [p] complex double: the sum of the partials
 };
 int launch_tap_gradient(int real_bytes, const TapGradLaunch &a, hipStream_t st);

@@ -14,7 +14,7 @@ BP: the backprojector (kernel.cu:68-177).  The adjoints are hand-written:
 
 With ``chunk`` set, neither pass holds a filtered or weighted copy of the
 whole stack: the forward pass filters and packs ``chunk`` projections at a time
-into the stored stack, and the backward pass recomputes q = W p per chunk
+into the stored stack, and the backward pass recomputes q = W p as it is read
 (per-angle-chunk recomputation).  The backward pass forward-projects all angles
 at once straight into the gradient buffer (one read of the volume gradient).
 """
@@ -84,15 +84,12 @@ def backward(st: Stages, proj, gvol, chunk=None, need_proj=True, need_taps=True)
     dh = None
     if need_taps:
         dh = np.zeros(st.p, np.float64)
-        for a0 in range(0, nang, chunk):
-            n = min(chunk, nang - a0)
-            if n == nang:
-                q = st.weight(proj.detach().clone())
-                gy = gproj
-            else:
-                q = st.weight(proj[:, a0:a0 + n, :].contiguous())
-                gy = gproj[:, a0:a0 + n, :].contiguous()
-            st.tap_gradient(q, gy, dh)
+        # q = W p is formed as the rows are read: a contiguous stack needs no copy
+        # and goes in one call
+        n = nang if proj.is_contiguous() else chunk
+        for a0 in range(0, nang, n):
+            q, gy = (x[:, a0:a0 + n, :].contiguous() for x in (proj.detach(), gproj))
+            st.tap_gradient(q, gy, dh, weight=True)
             del q, gy
     if not need_proj:
         return None, dh

@@ -133,15 +133,16 @@ class Stages:
                    "fdk_forward_project")
         return out
 
-    def tap_gradient(self, q, G, dh=None):
-        """Accumulates d<G, filter_h(q)>/dh into dh (numpy float64 [p])."""
+    def tap_gradient(self, q, G, dh=None, weight=False):
+        """Accumulates d<G, filter_h(q)>/dh into dh (numpy float64 [p]); weight: q
+        are projections, weighted as they are read."""
         _check_dev(q)
         _check_dev(G, tuple(q.shape))
         if dh is None:
             dh = np.zeros(self.p, np.float64)
-        _lib.check(self.L.fdk_tap_gradient(self.fbp.handle, _dtype_code(q), q.data_ptr(),
-                                           G.data_ptr(), q.shape[1], dh.ctypes.data, _stream()),
-                   "fdk_tap_gradient")
+        fn = self.L.fdk_tap_gradient_weighted if weight else self.L.fdk_tap_gradient
+        _lib.check(fn(self.fbp.handle, _dtype_code(q), q.data_ptr(), G.data_ptr(), q.shape[1],
+                      dh.ctypes.data, _stream()), "fdk_tap_gradient")
         return dh
 
     def phantom(self, ells: np.ndarray, ang0=0, nang=None, out=None, device="cuda"):
