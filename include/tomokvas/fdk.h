@@ -171,6 +171,15 @@ int fdk_filter(fdk_ctx *ctx, int dtype, void *d_sino, int nang, int weight, int 
 /* bytes of the stored stack for nang projections in storage `store_dtype`:
  * [nang][Nv][pitch] samples, pitch >= Nu + 68 (zero-padded rows) */
 size_t fdk_stack_bytes(fdk_ctx *ctx, int store_dtype, int nang);
+/* fdk_filter out of place, for nang projections from the angle that d_in points at of
+ * a stack [Nv][in_nang][Nu].  store_dtype < 0: rows [Nv][nang][Nu] into d_out, with
+ * weight 0, 1 (before the filter, W then F_h) or 2 (after it; with `adjoint` the
+ * transpose W F_h^T); d_out may be d_in when nang = in_nang.  store_dtype F32 or BF16
+ * (F32 data) or F64: weighted and filtered into the stored stack and scales that
+ * fdk_pack would write (weight 1, no adjoint, no d_maxabs). */
+int fdk_filter_into(fdk_ctx *ctx, int dtype, const void *d_in, int in_nang, int nang,
+                    int weight, int adjoint, int store_dtype, void *d_out, void *d_scales,
+                    uint32_t *d_maxabs, void *stream);
 /* repack filtered [Nv][nang][Nu] (F32 or F64) into the backprojector's stored
  * stack (16-byte aligned); FP16 stores value/scale with scale = maxabs/8192 per
  * projection (d_maxabs required), F32/BF16/F64 store the values (scale 1) */

@@ -276,3 +276,42 @@ def test_weighted_tap_gradient(torch, Nu, Nv, Nang):
             ref = O.tap_gradient(ogeom(g), st.weight(p.clone()).double().cpu().numpy(),
                                  G.double().cpu().numpy())
             assert np.abs(got - ref).max() <= (1e-5 if dt == torch.float32 else 1e-12) * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("Nu", [1, 3, 37, 300, 700, 1024, 2048, 3000])
+@pytest.mark.parametrize("store", [_lib.F32, _lib.BF16, _lib.F64])
+def test_filter_into_the_stored_stack(torch, Nu, store):
+    """Slices of a stack filtered straight into a stored stack, into rows, and with
+    the weight after the filter, against the filter, pack and weight in turn."""
+    Nv, Nang, cut = 5, 7, 3
+    g = scan(Nu, Nv, Nang, 8, 8, 8, D=max(2500.0, Nu))
+    st = stages(g)
+    dt = torch.float64 if store == _lib.F64 else torch.float32
+    gen = torch.Generator(device="cuda").manual_seed(Nu)
+    d = torch.randn(st.sino_shape(), device="cuda", generator=gen, dtype=dt)
+    say(f"filter into, Nu {Nu} storage {store}")
+    # a slice's rows are transformed in pairs of its own, so the slices are filtered
+    # one by one on both sides
+    ya, yb = (st.filter(x.contiguous(), weight=True) for x in (d[:, :cut], d[:, cut:]))
+    want, wscales = st.pack(d, store)
+    st.pack_into(ya, store, want, wscales, 0)
+    st.pack_into(yb, store, want, wscales, cut)
+    got = torch.full_like(want, 0x55)
+    scales = torch.zeros_like(wscales)
+    st.filter_store(d, store, got, scales, 0, 0, cut)
+    st.filter_store(d, store, got, scales, cut, cut)
+    n = (st.stack_bytes(store, 1) - st.stack_bytes(store, 0)) * Nang
+    assert torch.equal(got[:n], want[:n]) and torch.equal(scales, wscales)
+    rows = torch.empty(st.sino_shape(Nang - cut), device="cuda", dtype=dt)
+    m = torch.zeros(Nang - cut, dtype=torch.int32, device="cuda")
+    st.filter_into(d, rows, weight=1, ang0=cut, maxabs=m)
+    assert torch.equal(rows, yb)
+    if dt == torch.float32:
+        assert torch.equal(m.view(torch.float32), rows.abs().amax(dim=(0, 2)))
+    z = st.weight(st.filter(d.clone(), adjoint=True))
+    st.filter_into(d, d, weight=2, adjoint=True)
+    assert torch.equal(d, z)
+    with pytest.raises(ValueError):
+        st.filter_into(d, rows, ang0=cut + 1)
+    with pytest.raises(_lib.FDKError):
+        st.filter_store(d, _lib.F16, got, scales)

@@ -317,16 +317,19 @@ double out_scale(const fdk_ctx *c, int dtype)
 
 // The per-projection maxima that the filter leaves for the pack: only FP16
 // storage scales by them, so the other storage types filter without them.
+bool scaled_storage(int dtype) { return dtype == FDK_F16 || dtype == FDK_F16_PACKED; }
+
 unsigned *pack_maxabs(const fdk_ctx *c)
 {
-    return c->storage == FDK_F16 || c->storage == FDK_F16_PACKED ? c->d_maxabs : nullptr;
+    return scaled_storage(c->storage) ? c->d_maxabs : nullptr;
 }
 
-int stage_filter(fdk_ctx *c, int dtype, const void *in, void *out, int nang, int weight,
-                 int adjoint, unsigned *maxabs, hipStream_t st)
+tkv::FilterLaunch filter_launch(const fdk_ctx *c, int dtype, const void *in, int in_nang,
+                                void *out, int nang, int weight, int adjoint, unsigned *maxabs)
 {
     tkv::FilterLaunch L;
     L.in = in;
+    L.in_nang = in_nang;
     L.out = out;
     L.Nu = c->g.Nu;
     L.Nv = c->g.Nv;
@@ -342,7 +345,42 @@ int stage_filter(fdk_ctx *c, int dtype, const void *in, void *out, int nang, int
     L.conj = adjoint;
     L.tw = f64 ? (const void *)c->d_tw64 : (const void *)c->d_tw32;
     L.maxabs = maxabs;
-    return tkv::launch_filter(f64 ? 8 : 4, L, st);
+    return L;
+}
+
+int stage_filter(fdk_ctx *c, int dtype, const void *in, void *out, int nang, int weight,
+                 int adjoint, unsigned *maxabs, hipStream_t st)
+{
+    return tkv::launch_filter(
+        dtype == FDK_F64 ? 8 : 4,
+        filter_launch(c, dtype, in, nang, out, nang, weight, adjoint, maxabs), st);
+}
+
+// Projections weighted and filtered into the stored stack of a type that stores
+// them unscaled: no filtered rows in between.
+int stage_filter_store(fdk_ctx *c, int store_dtype, const void *in, int in_nang, int nang,
+                       void *stack, void *scales, hipStream_t st)
+{
+    const int dtype = store_dtype == FDK_F64 ? FDK_F64 : FDK_F32;
+    tkv::FilterLaunch L = filter_launch(c, dtype, in, in_nang, stack, nang, 1, 0, nullptr);
+    L.pitch = tkv::stack_pitch(c->g.Nu);
+    L.store_dtype = store_dtype;
+    L.scales = scales;
+    return tkv::launch_filter(dtype == FDK_F64 ? 8 : 4, L, st);
+}
+
+// FP32 projections into the engine's stored stack: FP16 needs the filtered
+// projections' maxima before it can store them, the other types don't
+int filter_and_pack(fdk_ctx *c, const float *in, float *filt, int nang, unsigned *maxabs,
+                    void *stack, float *scales, hipEvent_t between, hipStream_t st)
+{
+    int rc = maxabs ? stage_filter(c, FDK_F32, in, filt, nang, 1, 0, maxabs, st)
+                    : stage_filter_store(c, c->storage, in, nang, nang, stack, scales, st);
+    if (rc) return rc;
+    if (between) TKV_HIP(hipEventRecord(between, st));
+    if (!maxabs) return FDK_OK;
+    return tkv::launch_pack(FDK_F32, filt, c->g.Nu, c->g.Nv, nang, tkv::stack_pitch(c->g.Nu),
+                            maxabs, c->storage, stack, scales, st);
 }
 
 // Slices [z0, z0 + nz) of the volume into vol (nz < 0: every slice).
@@ -844,6 +882,9 @@ int fdk_set_storage(fdk_ctx *c, int dtype)
     if (c->initialized && dtype != c->storage) {
         int rc = ensure(&c->d_stack, c->cap_stack, fdk_stack_bytes(c, dtype, c->g.Nang),
                         "stored stack");
+        if (!rc && scaled_storage(dtype))
+            rc = ensure((void **)&c->d_filt, c->cap_filt,
+                        (size_t)c->g.Nu * c->g.Nv * c->g.Nang * sizeof(float), "filtered stack");
         if (rc) return rc;
     }
     c->storage = dtype;
@@ -877,7 +918,8 @@ int fdk_initialize(fdk_ctx *c)
     const size_t nvol = (size_t)g.Nx * g.Ny * g.Nz;
     const size_t slab = (size_t)g.Nx * g.Ny * g.B;
     if ((rc = ensure((void **)&c->d_sino, c->cap_sino, nsino * sizeof(float), "projection stack")) ||
-        (rc = ensure((void **)&c->d_filt, c->cap_filt, nsino * sizeof(float), "filtered stack")) ||
+        (scaled_storage(c->storage) && (rc = ensure((void **)&c->d_filt, c->cap_filt,
+                                           nsino * sizeof(float), "filtered stack"))) ||
         (rc = ensure(&c->d_stack, c->cap_stack, fdk_stack_bytes(c, c->storage, g.Nang),
                      "stored stack")) ||
         (rc = ensure((void **)&c->d_scales, c->cap_scales, g.Nang * sizeof(float), "scales")) ||
@@ -964,11 +1006,8 @@ int fdk_calculate_reconstruction(fdk_ctx *c, fdk_get_block_fn get_block, void *u
     if (maxabs && (rc = tkv::launch_zero_u32(maxabs, g.Nang, st))) return rc;
     TKV_HIP(hipEventRecord(c->ev[0], st));
     // cosine weight fused into the row filter (kernel.cu:807-808)
-    if ((rc = stage_filter(c, FDK_F32, c->d_sino, c->d_filt, g.Nang, 1, 0, maxabs, st)))
-        return rc;
-    TKV_HIP(hipEventRecord(c->ev[1], st));
-    if ((rc = tkv::launch_pack(FDK_F32, c->d_filt, g.Nu, g.Nv, g.Nang, tkv::stack_pitch(g.Nu),
-                               maxabs, c->storage, c->d_stack, c->d_scales, st)))
+    if ((rc = filter_and_pack(c, c->d_sino, c->d_filt, g.Nang, maxabs, c->d_stack, c->d_scales,
+                              c->ev[1], st)))
         return rc;
     TKV_HIP(hipEventRecord(c->ev[2], st));
     if (!get_block) {
@@ -1036,8 +1075,7 @@ int fdk_reconstruct_host(fdk_ctx *c, const float *host_sino, fdk_get_block_fn ge
     const tkv::Geometry &g = c->g;
     hipStream_t st = c->stream, cs = c->copy_stream;
     const size_t per_ang = (size_t)g.Nu * g.Nv;
-    const int pitch = tkv::stack_pitch(g.Nu);
-    const size_t stored = (size_t)sample_bytes(c->storage) * pitch * g.Nv;
+    const size_t stored = (size_t)sample_bytes(c->storage) * tkv::stack_pitch(g.Nu) * g.Nv;
     const std::vector<int> ab =
         c->volume_mode == FDK_VOLUME_STREAMED ? std::vector<int>{0, g.Nang} : angle_bounds(g.Nang);
     const int K = (int)ab.size() - 1;
@@ -1057,7 +1095,8 @@ int fdk_reconstruct_host(fdk_ctx *c, const float *host_sino, fdk_get_block_fn ge
     if ((rc = upload(0))) return rc;
     for (int k = 0; k < K; ++k) {
         const int a0 = ab[k], nc = ab[k + 1] - a0;
-        float *in = c->d_sino + (size_t)a0 * per_ang, *filt = c->d_filt + (size_t)a0 * per_ang;
+        float *in = c->d_sino + (size_t)a0 * per_ang;
+        float *filt = maxabs ? c->d_filt + (size_t)a0 * per_ang : nullptr;
         void *stack = (char *)c->d_stack + (size_t)a0 * stored;
         float *scales = c->d_scales + a0;
         // the chunk's filter and pack on the prep stream once it has landed,
@@ -1065,10 +1104,7 @@ int fdk_reconstruct_host(fdk_ctx *c, const float *host_sino, fdk_get_block_fn ge
         // backprojection on the compute stream once they are done
         TKV_HIP(hipStreamWaitEvent(ps, c->ev_up[k & 1], 0));
         unsigned *const mx = maxabs ? maxabs + a0 : nullptr;
-        if ((rc = stage_filter(c, FDK_F32, in, filt, nc, 1, 0, mx, ps)) ||
-            (rc = tkv::launch_pack(FDK_F32, filt, g.Nu, g.Nv, nc, pitch, mx, c->storage, stack,
-                                   scales, ps)))
-            break;
+        if ((rc = filter_and_pack(c, in, filt, nc, mx, stack, scales, nullptr, ps))) break;
         TKV_HIP(hipEventRecord(c->ev_f[k & 1], ps));
         TKV_HIP(hipStreamWaitEvent(st, c->ev_f[k & 1], 0));
         if (k + 1 < K || !get_block) {
@@ -1139,8 +1175,39 @@ int fdk_filter(fdk_ctx *c, int dtype, void *d_sino, int nang, int weight, int ad
     if (dtype != FDK_F32 && dtype != FDK_F64)
         return fail(FDK_ERR_INVALID_ARGUMENT, "filter: F32 or F64 data");
     if (nang < 0) return fail(FDK_ERR_INVALID_ARGUMENT, "filter: negative angle count");
-    return stage_filter(c, dtype, d_sino, d_sino, nang, weight, adjoint, d_maxabs,
+    return stage_filter(c, dtype, d_sino, d_sino, nang, weight != 0, adjoint, d_maxabs,
                         pick(c, stream));
+}
+
+int fdk_filter_into(fdk_ctx *c, int dtype, const void *d_in, int in_nang, int nang, int weight,
+                    int adjoint, int store_dtype, void *d_out, void *d_scales,
+                    uint32_t *d_maxabs, void *stream)
+{
+    int rc = need_prepared(c);
+    if (rc) return rc;
+    if (dtype != FDK_F32 && dtype != FDK_F64)
+        return fail(FDK_ERR_INVALID_ARGUMENT, "filter_into: F32 or F64 data");
+    if (nang < 0 || in_nang < nang)
+        return fail(FDK_ERR_INVALID_ARGUMENT, "filter_into: angles outside the projections");
+    if (weight < 0 || weight > 2)
+        return fail(FDK_ERR_INVALID_ARGUMENT, "filter_into: weight is 0, 1 or 2");
+    if (!d_in || !d_out) return fail(FDK_ERR_INVALID_ARGUMENT, "filter_into: null buffer");
+    if (store_dtype < 0) {
+        if (d_in == d_out && in_nang != nang)
+            return fail(FDK_ERR_INVALID_ARGUMENT, "filter_into: in place needs all the angles");
+        return tkv::launch_filter(
+            dtype == FDK_F64 ? 8 : 4,
+            filter_launch(c, dtype, d_in, in_nang, d_out, nang, weight, adjoint, d_maxabs),
+            pick(c, stream));
+    }
+    if (store_dtype != dtype && !(store_dtype == FDK_BF16 && dtype == FDK_F32))
+        return fail(FDK_ERR_INVALID_ARGUMENT, "filter_into: storage is the data's type or BF16");
+    if (weight != 1 || adjoint || d_maxabs || !d_scales)
+        return fail(FDK_ERR_INVALID_ARGUMENT, "filter_into: a stored stack is W then F_h");
+    if ((uintptr_t)d_out & 15)
+        return fail(FDK_ERR_INVALID_ARGUMENT, "filter_into: stored stack not 16-byte aligned");
+    return stage_filter_store(c, store_dtype, d_in, in_nang, nang, d_out, d_scales,
+                              pick(c, stream));
 }
 
 int fdk_pack(fdk_ctx *c, int dtype_in, const void *d_filtered, int nang,

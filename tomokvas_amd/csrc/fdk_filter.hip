@@ -363,9 +363,29 @@ struct Passes {
     }
 };
 
-template <typename R, typename PL, int WAVES>
+// one stored sample
+struct bf16_t;
+template <typename Out>
+struct Elem {
+    using T = Out;
+    static __device__ __forceinline__ Out make(Out x) { return x; }
+};
+template <>
+struct Elem<bf16_t> {
+    using T = unsigned short;
+    static __device__ __forceinline__ T make(float x)
+    {
+        return __bfloat16_as_ushort(__float2bfloat16(x));
+    }
+};
+
+// Where the filtered rows go: Out = R and pitch 0, rows [v][angle][Nu] again (out
+// may be in); else the stored stack [angle][v][pitch] of Out with zeros from Nu on
+// and scales of 1, which spares unscaled storage the pack's pass over the rows.
+template <typename R, typename PL, int WAVES, typename Out>
 __global__ void __launch_bounds__(PL::BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES)))
-    filter_kernel(const R *in, R *out, int Nu, int Nv, int nang, int weight, R cX, R cZ, R D,
+    filter_kernel(const R *in, long long in_v, typename Elem<Out>::T *out, int pitch, R *scales,
+                  int Nu, int Nv, int nang, int weight, R cX, R cZ, R D,
                   const R *__restrict__ Hre, const R *__restrict__ Him, int conj,
                   const cpx<R> *__restrict__ tw, unsigned *__restrict__ maxabs)
 {
@@ -373,8 +393,10 @@ __global__ void __launch_bounds__(PL::BLOCK) __attribute__((amdgpu_waves_per_eu(
     constexpr int E = PL::E;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int tid = threadIdx.x;
-    const int f = tid / PL::TPT;          // transform within the workgroup
-    const int t = tid - f * PL::TPT;      // thread within the transform
+    // transform within the workgroup (one per wave or more: a scalar, and with it
+    // the rows' addresses), thread within the transform
+    const int f = PL::TPT >= 64 ? __builtin_amdgcn_readfirstlane(tid / PL::TPT) : tid / PL::TPT;
+    const int t = tid - f * PL::TPT;
     cpx<R> *s = reinterpret_cast<cpx<R> *>(smem_raw) + f * Pad<R, PL>::SIZE;
     const long long rows = (long long)Nv * nang;
     const long long rA = 2 * ((long long)blockIdx.x * PL::NT + f);
@@ -382,8 +404,10 @@ __global__ void __launch_bounds__(PL::BLOCK) __attribute__((amdgpu_waves_per_eu(
     const bool hasA = rA < rows, hasB = rB < rows;
     const int vA = hasA ? (int)(rA / nang) : 0;
     const int vB = hasB ? (int)(rB / nang) : 0;
-    const R *inA = in + (hasA ? rA : 0) * Nu;
-    const R *inB = in + (hasB ? rB : 0) * Nu;
+    const int aA = hasA ? (int)(rA - (long long)vA * nang) : 0;
+    const int aB = hasB ? (int)(rB - (long long)vB * nang) : 0;
+    const R *inA = in + vA * in_v + (long long)aA * Nu;
+    const R *inB = in + vB * in_v + (long long)aB * Nu;
 
     cpx<R> reg[E];
     // first pass inputs straight from HBM: two rows as (re, im), optional
@@ -414,7 +438,7 @@ __global__ void __launch_bounds__(PL::BLOCK) __attribute__((amdgpu_waves_per_eu(
             if (m < MH) {
                 a = hasA && n < Nu ? la[m] : (R)0;
                 c = hasB && n < Nu ? lc[m] : (R)0;
-                if (weight) {   // finite for every n < P/2; zeros stay zero
+                if (weight == 1) {   // finite for every n < P/2; zeros stay zero
                     const R wa = cos_weight<R>(n, vA, cX, cZ, D);
                     a *= wa;
                     if (same_v)
@@ -469,8 +493,9 @@ __global__ void __launch_bounds__(PL::BLOCK) __attribute__((amdgpu_waves_per_eu(
     // crop to Nu straight to HBM, per-projection max |value|
     using DI = DFT<R, PL::RLAST, true>;
     R mA = 0, mB = 0;
-    R *outA = out + (hasA ? rA : 0) * Nu;
-    R *outB = out + (hasB ? rB : 0) * Nu;
+    using EL = Elem<Out>;
+    typename EL::T *outA = out + (pitch ? ((size_t)aA * Nv + vA) * pitch : (size_t)(hasA ? rA : 0) * Nu);
+    typename EL::T *outB = out + (pitch ? ((size_t)aB * Nv + vB) * pitch : (size_t)(hasB ? rB : 0) * Nu);
     // (outputs m >= RLAST/2, n >= P/2 >= Nu, are cropped: their arithmetic in
     // the last pass is dead and removed at compile time)
 #pragma unroll
@@ -481,13 +506,26 @@ __global__ void __launch_bounds__(PL::BLOCK) __attribute__((amdgpu_waves_per_eu(
             const int n = i + m * (P / PL::RLAST);
             if (n < Nu) {
                 cpx<R> z = reg[b * PL::RLAST + DI::pos(m)];
-                if (hasA) outA[n] = z.x;
-                if (hasB) outB[n] = z.y;
+                if (weight == 2) {   // the transpose: weighted after the filter
+                    const R wa = cos_weight<R>(n, vA, cX, cZ, D);
+                    z.x *= wa;
+                    z.y *= same_v ? wa : cos_weight<R>(n, vB, cX, cZ, D);
+                }
+                if (hasA) outA[n] = EL::make(z.x);
+                if (hasB) outB[n] = EL::make(z.y);
                 R ax = z.x < 0 ? -z.x : z.x, ay = z.y < 0 ? -z.y : z.y;
                 mA = ax > mA ? ax : mA;
                 mB = ay > mB ? ay : mB;
             }
         }
+    }
+    for (int n = Nu + t; n < pitch; n += PL::TPT) {
+        if (hasA) outA[n] = EL::make((R)0);
+        if (hasB) outB[n] = EL::make((R)0);
+    }
+    if (scales && t == 0) {
+        if (hasA && vA == 0) scales[aA] = (R)1;
+        if (hasB && vB == 0) scales[aB] = (R)1;
     }
     if (maxabs) {
         // the workgroup's rows are 2 NT consecutive ones, so their maxima lie side
@@ -514,8 +552,8 @@ __global__ void __launch_bounds__(PL::BLOCK) __attribute__((amdgpu_waves_per_eu(
     }
 }
 
-template <typename R, typename PL, int WAVES>
-static int launch_filter_plan(const FilterLaunch &a, hipStream_t st)
+template <typename R, typename PL, int WAVES, typename Out>
+static int launch_filter_out(const FilterLaunch &a, hipStream_t st)
 {
     constexpr int P = PL::P;
     long long rows = (long long)a.Nv * a.nang;
@@ -527,7 +565,7 @@ static int launch_filter_plan(const FilterLaunch &a, hipStream_t st)
     size_t lds = PL::NPASS > 1 || PL::RFIRST != PL::RLAST
                      ? sizeof(cpx<R>) * (size_t)PL::NT * Pad<R, PL>::SIZE
                      : 0;
-    auto kern = filter_kernel<R, PL, WAVES>;
+    auto kern = filter_kernel<R, PL, WAVES, Out>;
     // beyond 64 KiB (one transform of p = 16384 in FP32, 8192 in FP64) the
     // workgroup takes up to the 160 KiB of LDS of a gfx950 CU
     if (lds > 163840) return fail(FDK_ERR_UNSUPPORTED, "filter: transform does not fit LDS");
@@ -535,11 +573,20 @@ static int launch_filter_plan(const FilterLaunch &a, hipStream_t st)
         TKV_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)lds));
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(PL::BLOCK), lds, st, (const R *)a.in,
-                       (R *)a.out, a.Nu, a.Nv, a.nang, a.weight, (R)a.cX, (R)a.cZ, (R)a.D,
+                       (long long)a.in_nang * a.Nu, (typename Elem<Out>::T *)a.out, a.pitch,
+                       (R *)a.scales, a.Nu, a.Nv, a.nang, a.weight, (R)a.cX, (R)a.cZ, (R)a.D,
                        (const R *)a.Hre, (const R *)a.Him, a.conj, (const cpx<R> *)a.tw,
                        a.maxabs);
     TKV_HIP(hipGetLastError());
     return FDK_OK;
+}
+
+template <typename R, typename PL, int WAVES>
+static int launch_filter_plan(const FilterLaunch &a, hipStream_t st)
+{
+    if constexpr (sizeof(R) == 4)
+        if (a.pitch && a.store_dtype == FDK_BF16) return launch_filter_out<R, PL, WAVES, bf16_t>(a, st);
+    return launch_filter_out<R, PL, WAVES, R>(a, st);
 }
 
 // radix 16 over 256 threads, at most 16 values per thread: FP32 p = 8192 one
@@ -886,7 +933,6 @@ struct Pack4<double> {
     }
 };
 struct f16_t;
-struct bf16_t;
 template <>
 struct Pack4<f16_t> {
     using V = uint2;

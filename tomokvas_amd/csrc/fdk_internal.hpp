@@ -82,10 +82,14 @@ inline bool grid_fits(long long blocks, int threads)
 }
 
 struct FilterLaunch {
-    const void *in;         // [rows][Nu] rows = Nv * nang, Real
-    void *out;              // may alias in
+    const void *in;         // nang projections of [Nv][in_nang][Nu], Real
+    int in_nang;
+    void *out;              // [Nv][nang][Nu], may alias in when in_nang = nang
+    int pitch = 0;          // or the stored stack [nang][Nv][pitch], of
+    int store_dtype = 0;    // store_dtype (Real's own type or BF16), with
+    void *scales = nullptr; // scales of 1
     int Nu, Nv, nang, p;
-    int weight;             // fuse the cosine pre-weight into the load
+    int weight;             // 1: cosine weight on load, 2: on the filtered rows
     float cX, cZ, D;
     const void *Hre, *Him;  // device spectrum [p] (Real), Him may be null (real H)
     int conj;               // multiply by conj(H) (adjoint)

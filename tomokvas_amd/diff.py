@@ -9,13 +9,12 @@ learnable spatial taps h, spectrum H = DFT_p(h) (the reference's fConvolution,
 kernel.cu:557-781, with the Ram-Lak taps of kernel.cu:783-802 replaced by h);
 BP: the backprojector (kernel.cu:68-177).  The adjoints are hand-written:
 
-    dL/dp = W F_h^T BP^T g        fdk_forward_project, fdk_filter(adjoint=1), fdk_weight
-    dL/dh = d<BP^T g, F_h q>/dh   fdk_tap_gradient, q = W p
+    dL/dp = W F_h^T BP^T g        fdk_forward_project, fdk_filter_into(adjoint)
+    dL/dh = d<BP^T g, F_h q>/dh   fdk_tap_gradient_weighted, q = W p
 
 With ``chunk`` set, neither pass holds a filtered or weighted copy of the
 whole stack: the forward pass filters and packs ``chunk`` projections at a time
-into the stored stack, and the backward pass recomputes q = W p as it is read
-(per-angle-chunk recomputation).  The backward pass forward-projects all angles
+into the stored stack, and the backward pass recomputes q = W p as it is read.  The backward pass forward-projects all angles
 at once straight into the gradient buffer (one read of the volume gradient).
 """
 from __future__ import annotations
@@ -53,6 +52,11 @@ def ramlak_taps(st: Stages) -> np.ndarray:
     return np.real(np.fft.ifft(H))
 
 
+def _slice(x, a0, n):
+    """Projections [a0, a0 + n) of a stack that is not contiguous, as a copy."""
+    return x[:, a0:a0 + n, :].contiguous() if n < x.shape[1] else x.detach().clone()
+
+
 def forward(st: Stages, proj, storage=_lib.F32, chunk=None):
     """FDK of proj [Nv][Nang][Nu] with the context's filter; returns the volume.
     FP64 input uses FP64 throughout; FP32 input is stored as `storage`."""
@@ -63,11 +67,17 @@ def forward(st: Stages, proj, storage=_lib.F32, chunk=None):
     stack = torch.empty(st.stack_bytes(store), dtype=torch.uint8, device=proj.device)
     scales = torch.empty(nang, dtype=torch.float64 if store == _lib.F64 else torch.float32,
                          device=proj.device)
+    whole = proj.is_contiguous()      # slices are read in place
+    scaled = store in (_lib.F16, _lib.F16_PACKED)
     for a0 in range(0, nang, chunk):
         n = min(chunk, nang - a0)
-        y = proj[:, a0:a0 + n, :].contiguous() if n < nang else proj.detach().clone()
+        src, s0 = (proj.detach(), a0) if whole else (_slice(proj, a0, n), 0)
+        if not scaled:                                # W then F_h, straight into the stack
+            st.filter_store(src, store, stack, scales, a0, s0, n)
+            continue
         maxabs = torch.zeros(n, dtype=torch.int32, device=proj.device)
-        st.filter(y, weight=True, maxabs=maxabs)      # W then F_h, per-projection max |y|
+        y = torch.empty(st.sino_shape(n), dtype=proj.dtype, device=proj.device)
+        st.filter_into(src, y, weight=1, ang0=s0, maxabs=maxabs)   # per-projection max |y|
         st.pack_into(y, store, stack, scales, a0, maxabs)
         del y
     return st.backproject(stack, store, scales)
@@ -86,13 +96,14 @@ def backward(st: Stages, proj, gvol, chunk=None, need_proj=True, need_taps=True)
         dh = np.zeros(st.p, np.float64)
         # q = W p is formed as the rows are read: a contiguous stack needs no copy
         # and goes in one call
-        n = nang if proj.is_contiguous() else chunk
-        for a0 in range(0, nang, n):
-            q, gy = (x[:, a0:a0 + n, :].contiguous() for x in (proj.detach(), gproj))
-            st.tap_gradient(q, gy, dh, weight=True)
-            del q, gy
+        if proj.is_contiguous():
+            st.tap_gradient(proj.detach(), gproj, dh, weight=True)
+        else:
+            for a0 in range(0, nang, chunk):
+                n = min(chunk, nang - a0)
+                gy = gproj if n == nang else _slice(gproj, a0, n)
+                st.tap_gradient(_slice(proj, a0, n), gy, dh, weight=True)
     if not need_proj:
         return None, dh
-    st.filter(gproj, adjoint=True)                     # F_h^T, in place
-    st.weight(gproj)                                   # W^T = W
+    st.filter_into(gproj, gproj, weight=2, adjoint=True)   # W F_h^T, in place
     return gproj, dh

@@ -73,6 +73,41 @@ class Stages:
                                      int(weight), int(adjoint), mp, _stream()), "fdk_filter")
         return sino
 
+    def filter_into(self, sino, out, weight=0, adjoint=False, ang0=0, maxabs=None):
+        """Projections [ang0, ang0 + n) of sino filtered into out [Nv][n][Nu] (sino
+        itself for all of them); weight 1: before the filter, 2: after it."""
+        _check_dev(sino)
+        _check_dev(out, (self.Nv, out.shape[1], self.Nu))
+        n = out.shape[1]
+        if out.dtype != sino.dtype or ang0 < 0 or ang0 + n > sino.shape[1] or \
+                tuple(sino.shape) != self.sino_shape(sino.shape[1]):
+            raise ValueError("filter_into: projections outside the stack, or of another type")
+        mp = None
+        if maxabs is not None:
+            _check_dev(maxabs, (n,))
+            mp = maxabs.data_ptr()
+        self._filter_into(sino, ang0, n, weight, adjoint, -1, out.data_ptr(), None, mp)
+        return out
+
+    def filter_store(self, sino, store_dtype, stack, scales, ang0=0, src0=0, n=None):
+        """Projections [src0, src0 + n) of sino, weighted and filtered, into projections
+        [ang0, ang0 + n) of a stored stack (F32 or BF16 for F32 data, or F64)."""
+        _check_dev(sino)
+        n = sino.shape[1] - src0 if n is None else n
+        per = self.stack_bytes(store_dtype, 1) - self.stack_bytes(store_dtype, 0)
+        if min(ang0, src0, n) < 0 or ang0 + n > scales.numel() or src0 + n > sino.shape[1] or \
+                tuple(sino.shape) != self.sino_shape(sino.shape[1]) or \
+                stack.numel() < self.stack_bytes(store_dtype, ang0 + n):
+            raise ValueError("filter_store: projections outside the stack")
+        self._filter_into(sino, src0, n, 1, False, store_dtype, stack.data_ptr() + ang0 * per,
+                          scales.data_ptr() + ang0 * scales.element_size(), None)
+
+    def _filter_into(self, sino, ang0, n, weight, adjoint, store, out, scales, maxabs):
+        _lib.check(self.L.fdk_filter_into(self.fbp.handle, _dtype_code(sino),
+                                          sino.data_ptr() + ang0 * self.Nu * sino.element_size(),
+                                          sino.shape[1], n, weight, int(adjoint), store, out,
+                                          scales, maxabs, _stream()), "fdk_filter_into")
+
     def stack_bytes(self, store_dtype, nang=None):
         return self.L.fdk_stack_bytes(self.fbp.handle, store_dtype,
                                       self.Nang if nang is None else nang)
