@@ -77,6 +77,11 @@ FP_CASES = {
     "two": dict(Nu=140, Nv=140, Nang=8, Nx=64, Ny=64, Nz=64, D=900.0, scale=2.0),
     "half": dict(Nu=48, Nv=40, Nang=9, Nx=70, Ny=40, Nz=67, D=300.0, scale=0.5),
     "four": dict(Nu=160, Nv=160, Nang=6, Nx=40, Ny=40, Nz=40, D=900.0, scale=4.0),
+    # footprints of both boxes' memory at every angle or at some, with the others
+    # in one box or in HBM
+    "large": dict(Nu=170, Nv=190, Nang=9, Nx=64, Ny=64, Nz=70, D=420.0, scale=2.0),
+    "larger": dict(Nu=180, Nv=240, Nang=9, Nx=64, Ny=60, Nz=64, D=260.0, scale=2.2),
+    "mixed": dict(Nu=150, Nv=170, Nang=30, Nx=66, Ny=66, Nz=64, D=700.0, scale=1.9),
 }
 
 

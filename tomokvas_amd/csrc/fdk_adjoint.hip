@@ -129,6 +129,9 @@ constexpr int FP_W = 108;
 constexpr int FP_H = 160;
 constexpr int FP_P = FP_W + 1;                  // odd pitch: the rows of one column
                                                 // fall in distinct LDS banks
+// a footprint beyond that takes the memory of both boxes as one of 136 x 254
+constexpr int FP_W2 = 136, FP_P2 = FP_W2 + 1, FP_H2 = 2 * FP_P * FP_H / FP_P2;
+constexpr int BOX_LARGE = 0x40000;              // flag beside such a footprint's width
 constexpr int FP_XP = FP_T + 1;                 // row pitch of the voxel transposition
 static_assert(FP_T / 2 * FP_ZR * FP_XP <= 2 * FP_P * FP_H, "voxel transposition beyond the boxes");
 
@@ -172,7 +175,10 @@ __device__ __forceinline__ float lane_f32(float x, int lane)
 // ms now).  The one workgroup of 16 waves fills a CU, so there are two boxes and
 // one barrier per angle, and odd waves flush the last angle's box after this
 // angle's splats, even waves before them: the flush's LDS and memory latency
-// then overlaps other waves' splats.
+// then overlaps other waves' splats.  An angle whose footprint needs the memory of
+// both boxes has its splats and its flush one after the other; straight into HBM
+// its splats cost 12 times as much (332 x 326 x 164 voxels, 35 projections at two
+// samples per voxel and magnifications up to 1.22: 0.69 ms, 8.1 with those in HBM).
 __global__ void __launch_bounds__(64 * FP_WAVES) fp_lds_kernel(FPArgs<float> a)
 {
     extern __shared__ __align__(16) int fp_mem[];
@@ -283,7 +289,7 @@ __global__ void __launch_bounds__(64 * FP_WAVES) fp_lds_kernel(FPArgs<float> a)
     int *cur = box;                       // the box of this angle
     // the last angle splatted and not yet flushed (fb < 0: none): its box, first
     // column and row, columns (taps reach one past the last) and cells
-    int fb = -1, fu0 = 0, fv0 = 0, fw = 1, fn = 0;
+    int fb = -1, fu0 = 0, fv0 = 0, fw = 1, fn = 0, fpitch = FP_P;
     int *fbox = box;
     // flush and clear: one global atomic per touched sample; the waves take
     // 64 consecutive cells of the box's used columns in turn, four at a time
@@ -295,15 +301,15 @@ __global__ void __launch_bounds__(64 * FP_WAVES) fp_lds_kernel(FPArgs<float> a)
             int t[4], rr[4], cc[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int q = q0 + i * 64 * FP_WAVES;   // < 2^15: exact in float
+                const int q = q0 + i * 64 * FP_WAVES;   // < 2^16: exact in float
                 rr[i] = (int)(((float)q + 0.5f) * winv);
                 cc[i] = q - rr[i] * fw;
-                t[i] = q < fn ? fbox[rr[i] * FP_P + cc[i]] : 0;
+                t[i] = q < fn ? fbox[rr[i] * fpitch + cc[i]] : 0;
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if (t[i] == 0) continue;
-                fbox[rr[i] * FP_P + cc[i]] = 0;
+                fbox[rr[i] * fpitch + cc[i]] = 0;
                 const int vr = fv0 + rr[i], uc = fu0 + cc[i];
                 if (vr < a.Nv && uc < a.Nu)
                     splat(out + (size_t)vr * rstride + uc, (float)t[i] * fxinv);
@@ -316,8 +322,14 @@ __global__ void __launch_bounds__(64 * FP_WAVES) fp_lds_kernel(FPArgs<float> a)
             __syncthreads();
             if (wave == 0 && b + lane < b1) {
                 const float c = a.ang[2 * (b + lane)], s = a.ang[2 * (b + lane) + 1];
-                boxes[lane] = footprint(c, s, cx0, cx1, cy0, cy1, azlo, azhi, a.cX, a.cZ, a.D, a.Nu,
-                                        a.Nv, FP_H, FP_W);
+                int4 q = footprint(c, s, cx0, cx1, cy0, cy1, azlo, azhi, a.cX, a.cZ, a.D, a.Nu,
+                                   a.Nv, FP_H, FP_W);
+                if (q.z < 0) {
+                    q = footprint(c, s, cx0, cx1, cy0, cy1, azlo, azhi, a.cX, a.cZ, a.D, a.Nu,
+                                  a.Nv, FP_H2, FP_W2);
+                    if (q.z > 0) q.z |= BOX_LARGE;
+                }
+                boxes[lane] = q;
                 angs[lane] = make_float2(c, s);
             }
             __syncthreads();
@@ -348,14 +360,20 @@ __global__ void __launch_bounds__(64 * FP_WAVES) fp_lds_kernel(FPArgs<float> a)
             // splat into the LDS box; taps with zero weight past the
             // detector's last row or column land inside the box and are
             // dropped at the flush
-            const bool inner = bw & BOX_INNER_V;
+            const bool inner = bw & BOX_INNER_V, large = bw & BOX_LARGE;
+            if (large) {
+                flush();
+                __syncthreads();          // both boxes are clear
+                cur = box;
+            }
             char *lds = (char *)cur;
             // LDS byte offset of the column's sample in detector row 0; the
             // weights in units of 1/fxs
-            const int cb = (iu - bu0) * 4 - bv0 * (4 * FP_P);
+            const int cb = (iu - bu0) * 4 - bv0 * 4 * (large ? FP_P2 : FP_P);
             const float ws0 = w0 * fxs, ws1 = w1 * fxs;
-            auto splats = [&](auto inner_tag) {
+            auto splats = [&](auto inner_tag, auto pitch_tag) {
                 constexpr bool INNER = decltype(inner_tag)::value;
+                constexpr int P = decltype(pitch_tag)::value;
 #pragma unroll
                 for (int j = 0; j < 64; ++j) {
                     if (!((j < 32 ? todo_lo : todo_hi) & (1u << (j & 31)))) continue;   // scalar
@@ -364,19 +382,25 @@ __global__ void __launch_bounds__(64 * FP_WAVES) fp_lds_kernel(FPArgs<float> a)
                     const int cbj = __builtin_amdgcn_readlane(cb, j);
                     if (INNER || (v >= 0.f && v <= a.vmax)) {
                         const float fv = __builtin_amdgcn_fractf(v);
-                        int *p0 = (int *)(lds + (int)__umul24((unsigned)(int)v, rowb) + cbj);
+                        int *p0 = (int *)(lds + (int)__umul24((unsigned)(int)v,
+                                                              P == FP_P ? rowb : 4u * P) + cbj);
                         const int t0 = round_half_up(s0 * fv), t1 = round_half_up(s1 * fv);
                         atomicAdd(p0, __float2int_rn(s0) - t0);
                         atomicAdd(p0 + 1, __float2int_rn(s1) - t1);
-                        atomicAdd(p0 + FP_P, t0);
-                        atomicAdd(p0 + FP_P + 1, t1);
+                        atomicAdd(p0 + P, t0);
+                        atomicAdd(p0 + P + 1, t1);
                     }
                 }
             };
-            if (!(wave & 1)) flush();
-            if (inner) splats(std::true_type{});
-            else splats(std::false_type{});
-            if (wave & 1) flush();
+            using pitch_t = std::integral_constant<int, FP_P>;
+            if (large) {
+                splats(std::false_type{}, std::integral_constant<int, FP_P2>{});
+            } else {
+                if (!(wave & 1)) flush();
+                if (inner) splats(std::true_type{}, pitch_t{});
+                else splats(std::false_type{}, pitch_t{});
+                if (wave & 1) flush();
+            }
             // the box splatted last is complete and the other one clear
             __syncthreads();
             fb = b;
@@ -385,7 +409,15 @@ __global__ void __launch_bounds__(64 * FP_WAVES) fp_lds_kernel(FPArgs<float> a)
             fv0 = bv0;
             fw = (bw & 0xffff) + 1;
             fn = fw * (bh + 1);
-            cur = cur == box ? box + FP_H * FP_P : box;
+            if (large) {
+                fpitch = FP_P2;
+                flush();
+                __syncthreads();          // both boxes are clear again
+                fpitch = FP_P;
+                fb = -1;
+            } else {
+                cur = cur == box ? box + FP_H * FP_P : box;
+            }
         } else {
             // box beyond the LDS tile: splat straight into HBM
 #pragma unroll
