@@ -50,9 +50,8 @@
 // 1800 x 2048^2):
 //   TKV_BP_ZR_F32 / _F16 / _BF16 / _F16P  slices per thread (register z-run)
 //                                  per storage type (FP64 uses 8)
-//   TKV_BP_LB                      LDS gathers per lane issued together
-//   TKV_BP_GROUP_FENCE             1: no instruction moves between groups of
-//                                  LB gathers
+//   TKV_BP_LB                      packed FP16: LDS gathers per lane issued
+//                                  together
 //   TKV_BP_BOXP_F32 / _F16P        LDS row pitch of the staged box in 32-bit
 //                                  words (>= 64, multiple of 4): rows of one
 //                                  column fall in different banks (FP32 samples;
@@ -71,10 +70,6 @@
 #endif
 #ifndef TKV_BP_LB
 #define TKV_BP_LB 4
-#endif
-// TKV_BP_GROUP_FENCE: the compiler schedules each group of LB gathers on its own
-#ifndef TKV_BP_GROUP_FENCE
-#define TKV_BP_GROUP_FENCE 1
 #endif
 #ifndef TKV_BP_BOXP_F32
 #define TKV_BP_BOXP_F32 80
@@ -198,40 +193,39 @@ __device__ __forceinline__ float rfract(float x) { return __builtin_amdgcn_fract
 template <>
 __device__ __forceinline__ double rfract(double x) { return __builtin_amdgcn_fract(x); }
 
-// ---- LDS gathers of one angle for LB slices of a thread's z-run ----------------------
-// acc[k] += W * bilinear(box; u, v_k) with v_k = az[k]*Uv + cz; colb is the
-// byte offset of the thread's column minus that of the box's first row.
+// ---- LDS gather of one angle for one slice of a thread's z-run ------------------------
+// acc[k] += W * bilinear(box; u, v_k) with v_k = az[k]*Uv + cz; col is where the
+// thread's column would lie in detector row 0 (a pointer, so that a sample's
+// address is one multiply-add from the row).
 // FAST: every v_k of every lane of the wave lies inside [0.01, Nv-1.01].
-template <bool FAST, int LB, int P>
-__device__ __forceinline__ void gather_lds(float *acc, const float *az, const float *box,
-                                           float Uv, float cz, int colb, float wu0, float wu1,
-                                           float vmax)
-{
-    const char *lds = (const char *)box;
-    float c0[LB], c1[LB];
-    bool okk[LB];
-#pragma unroll
-    for (int k = 0; k < LB; ++k) {
-        const float v = fmaf(az[k], Uv, cz);
-        const float fv = __builtin_amdgcn_fractf(v);
-        bool ok = true;
-        int off = (int)__umul24((unsigned)(int)v, 4u * P) + colb;   // v >= 0 where used
+template <bool FAST, int P>
+struct LdsGather {
+    float fv, q00, q01, q10, q11;
+    bool ok;
+    __device__ __forceinline__ void issue(float az, const float *box, float Uv, float cz,
+                                          const char *col, float vmax)
+    {
+        const float v = fmaf(az, Uv, cz);
+        fv = __builtin_amdgcn_fractf(v);
+        // v >= 0 where used
+        const float *p0 = (const float *)(col + (int)__umul24((unsigned)(int)v, 4u * P));
+        ok = true;
         if (!FAST) {
             ok = v >= 0.f && v <= vmax;
-            off = ok ? off : 0;
+            p0 = ok ? p0 : box;
         }
-        const float *p0 = (const float *)(lds + off);
-        const float q00 = p0[0], q01 = p0[1];
-        const float q10 = p0[P], q11 = p0[P + 1];
-        c0[k] = fmaf(fv, q10 - q00, q00);
-        c1[k] = fmaf(fv, q11 - q01, q01);
-        okk[k] = ok;
+        q00 = p0[0];
+        q01 = p0[1];
+        q10 = p0[P];
+        q11 = p0[P + 1];
     }
     // taps outside the detector get zero weight (the staged values are finite)
-#pragma unroll
-    for (int k = 0; k < LB; ++k)
-        acc[k] = fmaf(okk[k] ? wu1 : 0.f, c1[k], fmaf(okk[k] ? wu0 : 0.f, c0[k], acc[k]));
-}
+    __device__ __forceinline__ float add(float acc, float wu0, float wu1) const
+    {
+        const float c0 = fmaf(fv, q10 - q00, q00), c1 = fmaf(fv, q11 - q01, q01);
+        return fmaf(ok ? wu1 : 0.f, c1, fmaf(ok ? wu0 : 0.f, c0, acc));
+    }
+};
 
 // FP16 pairs in LDS, packed-FP16 interpolation (FDK_F16_PACKED): the lerp
 // along v runs in packed FP16; the two column weights (FP16, normalised to at
@@ -239,11 +233,10 @@ __device__ __forceinline__ void gather_lds(float *acc, const float *az, const fl
 // FP32.
 template <bool FAST, int LB, int P>
 __device__ __forceinline__ void gather_pairs(float *acc, const float *az, const float *box,
-                                             float Uv, float cz, int colb, half2_t wuh,
+                                             float Uv, float cz, const char *col, half2_t wuh,
                                              float vmax)
 {
     static_assert(LB % 2 == 0, "fractions are converted in pairs");
-    const char *lds = (const char *)box;
     half2_t c[LB];
     bool okk[LB];
 #pragma unroll
@@ -257,13 +250,14 @@ __device__ __forceinline__ void gather_pairs(float *acc, const float *az, const 
         for (int j = 0; j < 2; ++j) {
             const float v = j ? vb : va;
             bool ok = true;
-            int off = (int)__umul24((unsigned)(int)v, 4u * P) + colb;   // v >= 0 where used
+            // v >= 0 where used
+            const float *p0 = (const float *)(col + (int)__umul24((unsigned)(int)v, 4u * P));
             if (!FAST) {
                 ok = v >= 0.f && v <= vmax;
-                off = ok ? off : 0;
+                p0 = ok ? p0 : box;
             }
-            const half2_t w0 = *(const half2_t *)(lds + off);
-            const half2_t w1 = *(const half2_t *)(lds + off + 4 * P);
+            const half2_t w0 = *(const half2_t *)p0;
+            const half2_t w1 = *(const half2_t *)(p0 + P);
             const half2_t f = j ? half2_t{fab.y, fab.y} : half2_t{fab.x, fab.x};
             c[k + j] = f * (w1 - w0) + w0;
             okk[k + j] = ok;
@@ -280,21 +274,33 @@ __device__ __forceinline__ void gather_pairs(float *acc, const float *az, const 
     }
 }
 
-// all ZR slices of a thread for one staged angle, LB gathers at a time
+// all ZR slices of a thread for one staged angle
 template <bool FAST, bool PAIRS, int ZR, int LB, int P>
 __device__ __forceinline__ void gather_run(float (&acc)[ZR], const float (&az)[ZR],
-                                           const float *box, float Uv, float cz, int colb,
-                                           float wu0, float wu1, half2_t wuh, float vmax)
+                                           const float *box, float Uv, float cz,
+                                           const char *col, float wu0, float wu1, half2_t wuh, float vmax)
 {
+    if constexpr (PAIRS) {
 #pragma unroll
-    for (int k0 = 0; k0 < ZR; k0 += LB) {
-        if constexpr (PAIRS)
-            gather_pairs<FAST, LB, P>(acc + k0, az + k0, box, Uv, cz, colb, wuh, vmax);
-        else
-            gather_lds<FAST, LB, P>(acc + k0, az + k0, box, Uv, cz, colb, wu0, wu1, vmax);
-#if TKV_BP_GROUP_FENCE
+        for (int k0 = 0; k0 < ZR; k0 += LB) {
+            gather_pairs<FAST, LB, P>(acc + k0, az + k0, box, Uv, cz, col, wuh, vmax);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    } else {
+        // one slice's samples are on their way while the slice before is added: left
+        // to itself the compiler waits for each slice's or holds those of several,
+        // which takes registers (256^3 from 360, FP32: 1.83 ms, 1.97 with a wait per
+        // slice, 1.87 with two slices together, 1.89 with two on their way)
+        LdsGather<FAST, P> g[2];
+        g[0].issue(az[0], box, Uv, cz, col, vmax);
+#pragma unroll
+        for (int k = 0; k < ZR; ++k) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (k + 1 < ZR) g[(k + 1) & 1].issue(az[k + 1], box, Uv, cz, col, vmax);
+            __builtin_amdgcn_sched_barrier(0);
+            acc[k] = g[k & 1].add(acc[k], wu0, wu1);
+        }
         __builtin_amdgcn_sched_barrier(0);
-#endif
     }
 }
 
@@ -582,10 +588,9 @@ __global__ void __launch_bounds__(256 * G) bp_kernel(BPArgs<typename Store<S>::R
                 const R wu1 = W * fu, wu0 = W - wu1;
                 half2_t wuh = {0, 0};
                 if constexpr (PACKED) wuh = half2_t{(_Float16)wu0, (_Float16)wu1};
-                // LDS byte offset of sample (row iv, column iu) is
-                // iv*4*P + colb
-                const int colb = iu * 4 - (qu * 4 + qv * (4 * P));
-                gather_run<FAST, ST::PAIRS, ZR, LB, P>(acc, az, boxmem, Uv, cz, colb, wu0, wu1,
+                // sample (row iv, column iu) lies at col + iv*4*P
+                const char *col = (const char *)boxmem + (iu * 4 - (qu * 4 + qv * (4 * P)));
+                gather_run<FAST, ST::PAIRS, ZR, LB, P>(acc, az, boxmem, Uv, cz, col, wu0, wu1,
                                                        wuh, a.vmax);
             };
             using fast_t = std::integral_constant<bool, true>;
@@ -605,29 +610,30 @@ __global__ void __launch_bounds__(256 * G) bp_kernel(BPArgs<typename Store<S>::R
                 const int ni = uniform_int(counts[slot * G + grp].x);
                 const int n = uniform_int(counts[slot * G + grp].y);
                 int mi = ni, me = n - ni;
-                for (int h = 0; h < G; ++h) {
-                    const int hi = uniform_int(counts[slot * G + h].x);
-                    mi = max(mi, hi);
-                    me = max(me, uniform_int(counts[slot * G + h].y) - hi);
-                }
-                const bool next = g + 1 < ngroups && uniform_int(counts[(slot ^ 1) * G + grp].y) > 0;
+                if constexpr (G > 1)
+                    for (int h = 0; h < G; ++h) {
+                        const int hi = uniform_int(counts[slot * G + h].x);
+                        mi = max(mi, hi);
+                        me = max(me, uniform_int(counts[slot * G + h].y) - hi);
+                    }
+                const int n1 = uniform_int(counts[(slot ^ 1) * G + grp].y);
                 const int base = slot * 64 + grp * (64 / G), base1 = base ^ 64;
                 if (!loading && n > 0) issue(ebox[base]);
-                loading = n > 0 && next;
-                // t-th of this group's entries [e0, e1), `most` steps; while one is
+                loading = n > 0 && g + 1 < ngroups && n1 > 0;
+                // this group's entries [e0, e1), in `most` steps; while one is
                 // gathered the next one's box is loaded (the next batch's first
                 // after the last)
                 auto run = [&](auto fast_tag, int e0, int e1, int most) {
-                    for (int t = 0; t < most; ++t) {
-                        const int j = e0 + t;
+                    for (int j = e0; G == 1 ? j < e1 : j < e0 + most; ++j) {
                         const bool mine = G == 1 || j < e1;
                         const int qu = bu0, qv = bv0, qh = bh;
                         const bool inner_u = bi & INNER_U;
+                        const int at = j + 1 < n ? base + j + 1 : base1;
                         const bool more = mine && (j + 1 < n || loading);
-                        const int4 e = ebox[j + 1 < n ? base + j + 1 : base1];
-                        const int at = base + (mine ? j : 0);
-                        const float wc = __int_as_float(ebox[at].w);
-                        const float2 ss = ess[at];
+                        const int4 e = ebox[at];            // (read, not used, if no more)
+                        const int own = base + (mine ? j : 0);
+                        const float wc = __int_as_float(ebox[own].w);
+                        const float2 ss = ess[own];
                         __syncthreads();   // every wave is done with the previous box
                         if (mine) stage.commit(boxmem, qh, tid);
                         __syncthreads();
