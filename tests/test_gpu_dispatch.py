@@ -137,6 +137,7 @@ BP_CASES = {
     "1056": dict(Nu=260, Nv=20, Nang=4, Nx=513, Ny=505, Nz=14, D=900.0, scale=0.5),
     "8192": dict(Nu=1100, Nv=40, Nang=5, Nx=1024, Ny=1020, Nz=20, D=2000.0),
     "8320": dict(Nu=1100, Nv=40, Nang=5, Nx=1025, Ny=1010, Nz=20, D=2000.0),
+    "8450, high boxes": dict(Nu=2140, Nv=60, Nang=4, Nx=1040, Ny=1030, Nz=20, D=7400.0, scale=2.05),
     "8450": dict(Nu=2300, Nv=70, Nang=3, Nx=1040, Ny=1040, Nz=17, D=3800.0, scale=2.2),
 }
 

@@ -26,7 +26,7 @@
 //    FP32 arithmetic on the decoded samples.  (FP16 pairs in the box, widened by
 //    mixed-precision FMAs, halve the LDS reads, but those FMAs issue at 1.1
 //    cycles per wave instruction and CU where plain FP32 arithmetic on vector
-//    registers takes 0.66: 38.9 against 37.6 ms for 512^3 from 900 x 1024^2.)
+//    registers takes 0.66: they are used for the highest boxes only.)
 //    FDK_F16_PACKED (opt-in) keeps FP16 pairs (q[c], q[c+1]) per 32-bit word,
 //    lerps in packed FP16 and weights with v_dot2 (FP16 fraction and column
 //    weights): faster, outside the precision form;
@@ -98,6 +98,7 @@ struct BPArgs {
     R *vol;
     int Nx, Ny, Nz, Nu, Nv, nang;
     R cX, cZ, D, umax, vmax, out_scale;
+    R one;                        // 1, at run time: see LdsGather
     double maskR2;
     int accumulate;
     int tiles_x, tiles_xy, nblocks;
@@ -105,12 +106,13 @@ struct BPArgs {
 };
 
 // ---- storage types ----------------------------------------------------------------
-// PAIRS: the LDS box holds FP16 sample pairs, interpolated in packed FP16 (else
-// FP32 samples)
+// PAIRS: the LDS box holds FP16 sample pairs, interpolated in packed FP16 or, MIX,
+// with FP32 fractions and weights in mixed-precision FMAs (else FP32 samples)
 struct st_f32;
 struct st_f16;
 struct st_bf16;
 struct st_f16p;
+struct st_f16m;
 struct st_f64;
 template <typename S>
 struct Store;
@@ -122,6 +124,7 @@ struct Store<st_f32> {
     static constexpr int ZR = TKV_BP_ZR_F32;
     static constexpr int P = TKV_BP_BOXP_F32;
     static constexpr bool PAIRS = false;
+    static constexpr bool MIX = false;
     static __device__ __forceinline__ float get(const char *p) { return *(const float *)p; }
     static __device__ __forceinline__ float half(unsigned, int) { return 0.f; }
 };
@@ -133,6 +136,7 @@ struct Store<st_f16> {
     static constexpr int ZR = TKV_BP_ZR_F16;
     static constexpr int P = TKV_BP_BOXP_F32;
     static constexpr bool PAIRS = false;
+    static constexpr bool MIX = false;
     static __device__ __forceinline__ float get(const char *p)
     {
         return __half2float(__ushort_as_half(*(const unsigned short *)p));
@@ -150,6 +154,7 @@ struct Store<st_bf16> {
     static constexpr int ZR = TKV_BP_ZR_BF16;
     static constexpr int P = TKV_BP_BOXP_F32;
     static constexpr bool PAIRS = false;
+    static constexpr bool MIX = false;
     static __device__ __forceinline__ float get(const char *p)
     {
         return __uint_as_float((unsigned)(*(const unsigned short *)p) << 16);
@@ -158,6 +163,12 @@ struct Store<st_bf16> {
     {
         return __uint_as_float(hi ? (w & 0xffff0000u) : (w << 16));
     }
+};
+template <>
+struct Store<st_f16m> : Store<st_f16> {
+    static constexpr int P = TKV_BP_BOXP_F16P;
+    static constexpr bool PAIRS = true;
+    static constexpr bool MIX = true;
 };
 template <>
 struct Store<st_f16p> : Store<st_f16> {
@@ -173,6 +184,7 @@ struct Store<st_f64> {
     static constexpr int ZR = 8;
     static constexpr int P = 64;   // unused: FP64 is gathered from HBM
     static constexpr bool PAIRS = false;
+    static constexpr bool MIX = false;
     static __device__ __forceinline__ double get(const char *p) { return *(const double *)p; }
     static __device__ __forceinline__ float half(unsigned, int) { return 0.f; }
 };
@@ -198,9 +210,16 @@ __device__ __forceinline__ double rfract(double x) { return __builtin_amdgcn_fra
 // thread's column would lie in detector row 0 (a pointer, so that a sample's
 // address is one multiply-add from the row).
 // FAST: every v_k of every lane of the wave lies inside [0.01, Nv-1.01].
-template <bool FAST, int P>
+// MIX: word (r, c) of the box holds the FP16 samples c and c+1 of row r.  Each
+// column's difference along v and its lerp are mixed-precision FMAs that read the
+// FP16 halves directly (v_fma_mix_f32; the product with `one`, 1 at run time, is
+// exact and the result rounds once to FP32), so they equal the FP32 operations on
+// the widened samples.
+template <bool FAST, bool MIX, int P>
 struct LdsGather {
-    float fv, q00, q01, q10, q11;
+    using Q = typename std::conditional<MIX, half2_t, float2>::type;
+    float fv;
+    Q q0, q1;   // rows iv and iv + 1
     bool ok;
     __device__ __forceinline__ void issue(float az, const float *box, float Uv, float cz,
                                           const char *col, float vmax)
@@ -214,15 +233,26 @@ struct LdsGather {
             ok = v >= 0.f && v <= vmax;
             p0 = ok ? p0 : box;
         }
-        q00 = p0[0];
-        q01 = p0[1];
-        q10 = p0[P];
-        q11 = p0[P + 1];
+        if constexpr (MIX) {
+            q0 = *(const half2_t *)p0;
+            q1 = *(const half2_t *)(p0 + P);
+        } else {
+            q0 = make_float2(p0[0], p0[1]);
+            q1 = make_float2(p0[P], p0[P + 1]);
+        }
     }
     // taps outside the detector get zero weight (the staged values are finite)
-    __device__ __forceinline__ float add(float acc, float wu0, float wu1) const
+    __device__ __forceinline__ float add(float acc, float wu0, float wu1, float one) const
     {
-        const float c0 = fmaf(fv, q10 - q00, q00), c1 = fmaf(fv, q11 - q01, q01);
+        float d0, d1;
+        if constexpr (MIX) {
+            d0 = fmaf((float)q1.x, one, -(float)q0.x);
+            d1 = fmaf((float)q1.y, one, -(float)q0.y);
+        } else {
+            d0 = q1.x - q0.x;
+            d1 = q1.y - q0.y;
+        }
+        const float c0 = fmaf(fv, d0, (float)q0.x), c1 = fmaf(fv, d1, (float)q0.y);
         return fmaf(ok ? wu1 : 0.f, c1, fmaf(ok ? wu0 : 0.f, c0, acc));
     }
 };
@@ -275,12 +305,13 @@ __device__ __forceinline__ void gather_pairs(float *acc, const float *az, const 
 }
 
 // all ZR slices of a thread for one staged angle
-template <bool FAST, bool PAIRS, int ZR, int LB, int P>
+template <bool FAST, typename ST, int ZR, int LB, int P>
 __device__ __forceinline__ void gather_run(float (&acc)[ZR], const float (&az)[ZR],
                                            const float *box, float Uv, float cz,
-                                           const char *col, float wu0, float wu1, half2_t wuh, float vmax)
+                                           const char *col, float wu0, float wu1, half2_t wuh, float vmax,
+                                           float one)
 {
-    if constexpr (PAIRS) {
+    if constexpr (ST::PAIRS && !ST::MIX) {
 #pragma unroll
         for (int k0 = 0; k0 < ZR; k0 += LB) {
             gather_pairs<FAST, LB, P>(acc + k0, az + k0, box, Uv, cz, col, wuh, vmax);
@@ -291,14 +322,14 @@ __device__ __forceinline__ void gather_run(float (&acc)[ZR], const float (&az)[Z
         // to itself the compiler waits for each slice's or holds those of several,
         // which takes registers (256^3 from 360, FP32: 1.83 ms, 1.97 with a wait per
         // slice, 1.87 with two slices together, 1.89 with two on their way)
-        LdsGather<FAST, P> g[2];
+        LdsGather<FAST, ST::MIX, P> g[2];
         g[0].issue(az[0], box, Uv, cz, col, vmax);
 #pragma unroll
         for (int k = 0; k < ZR; ++k) {
             __builtin_amdgcn_sched_barrier(0);
             if (k + 1 < ZR) g[(k + 1) & 1].issue(az[k + 1], box, Uv, cz, col, vmax);
             __builtin_amdgcn_sched_barrier(0);
-            acc[k] = g[k & 1].add(acc[k], wu0, wu1);
+            acc[k] = g[k & 1].add(acc[k], wu0, wu1, one);
         }
         __builtin_amdgcn_sched_barrier(0);
     }
@@ -461,7 +492,7 @@ __global__ void __launch_bounds__(256 * G) bp_kernel(BPArgs<typename Store<S>::R
     // packed FP16 carries the column weights in FP16: they are normalised by
     // the largest projection scale (rounded up to a power of two, g), so they
     // stay within [0, U^2], and the sums are multiplied by g at the end
-    constexpr bool PACKED = ST::PAIRS;
+    constexpr bool PACKED = ST::PAIRS && !ST::MIX;
     R wnorm = 1, wback = 1;
     if constexpr (PACKED) {
         float m = 0.f;
@@ -590,8 +621,8 @@ __global__ void __launch_bounds__(256 * G) bp_kernel(BPArgs<typename Store<S>::R
                 if constexpr (PACKED) wuh = half2_t{(_Float16)wu0, (_Float16)wu1};
                 // sample (row iv, column iu) lies at col + iv*4*P
                 const char *col = (const char *)boxmem + (iu * 4 - (qu * 4 + qv * (4 * P)));
-                gather_run<FAST, ST::PAIRS, ZR, LB, P>(acc, az, boxmem, Uv, cz, col, wu0, wu1,
-                                                       wuh, a.vmax);
+                gather_run<FAST, ST, ZR, LB, P>(acc, az, boxmem, Uv, cz, col, wu0, wu1, wuh,
+                                                a.vmax, a.one);
             };
             using fast_t = std::integral_constant<bool, true>;
             using edge_t = std::integral_constant<bool, false>;
@@ -833,6 +864,7 @@ static int launch_bp_z(const BPLaunch &L, hipStream_t st)
     a.umax = (R)(L.Nu - 1);
     a.vmax = (R)(L.Nv - 1);
     a.out_scale = (R)L.out_scale;
+    a.one = (R)1;
     a.maskR2 = L.maskR2;
     a.accumulate = L.accumulate;
     a.tiles_x = (L.Nx + 15) / 16;
@@ -859,7 +891,17 @@ static int launch_bp_t(const BPLaunch &L, hipStream_t st)
 {
     constexpr int ZR = Store<S>::ZR;
     const int z = L.shape.zrun, g = L.shape.groups;
-    if (z == ZR && g == 1) return launch_bp_z<S, ZR, 1>(L, st);
+    if (z == ZR && g == 1) {
+        // FP32 samples of a box of more than 80 rows leave room for four workgroups
+        // on a CU, FP16 pairs for five, and boxes that high are those of wide
+        // samplings and steep rays, whose gathers meet in the LDS banks: 512^3 at two
+        // samples per voxel from 150 angles, D 4096 (96 rows), 5.88 ms with pairs and
+        // 6.98 with FP32 samples.  With 80 rows the FP32 samples win: 512^3 from 900,
+        // D 10000, 38.8 and 36.8 ms; 512^2 x 300 at 1.8 samples from 150, 4.14 and 3.52.
+        if constexpr (std::is_same<S, st_f16>::value)
+            if (box_height<ZR>(L) > 80) return launch_bp_z<st_f16m, ZR, 1>(L, st);
+        return launch_bp_z<S, ZR, 1>(L, st);
+    }
     if constexpr (Store<S>::STAGED) {
         if (z == 8 && g == 4) return launch_bp_z<S, 8, 4>(L, st);
         if (z == 16 && g == 4) return launch_bp_z<S, 16, 4>(L, st);
