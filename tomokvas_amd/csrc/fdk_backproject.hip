@@ -780,7 +780,8 @@ static int native_zrun(int dtype)
 // whose blocks still don't fill the 256 CUs has 2 or 4 groups of 256 threads per
 // block, each gathering every 2nd or 4th angle from a box of its own; their sums
 // meet in LDS.  By blocks of 16^3 voxels; us for 32-slice (FP32: 24) runs, runs of
-// 16 with 1, 2, 4 groups, runs of 8 with 4 groups:
+// 16 with 1, 2, 4 groups, runs of 8 with 4 groups (before a slice's reads were
+// issued ahead, which takes another 3 to 6 % off most):
 //      8  32^3, 36 angles              60    45    33    30    22
 //     64  64^3, 90 angles             142   100    72    61    44
 //    108  96^2 x 40, 120, FP16        232   145    98    79    54
