@@ -338,19 +338,19 @@ __device__ __forceinline__ void gather_run(float (&acc)[ZR], const float (&az)[Z
 // Box staging in two steps, so the loads of the next angle's box fly while
 // the current angle is gathered: issue() loads rows [bv0, bv0+bh] of a
 // projection (the last is the +1 neighbour row; rows past the detector are
-// zero) x columns [bu0, bu0+64) into registers, 4 samples per lane and row,
+// zero) x columns [bu0, bu0+64) or the box's into registers, 4 samples per lane and row,
 // 16 lanes per row (columns past the row end read the stack's zero padding);
 // commit() writes them into the LDS box, widened to FP32; FP16 pair boxes hold
 // words (q[c], q[c+1]), the 4th word of a lane taking the next lane's first
 // sample (word 63 is never read).
-template <typename S, int ROWS>
+template <typename S, int ROWS, bool TRIM>
 struct BoxStage {
     using ST = Store<S>;
     static constexpr int PER = (ROWS + 15) / 16;   // rows per thread
     using Raw = typename std::conditional<ST::BYTES == 4, float4, uint2>::type;
     Raw raw[PER];
 
-    __device__ __forceinline__ void issue(const char *proj, int bu0, int bv0, int bh,
+    __device__ __forceinline__ void issue(const char *proj, int bu0, int bv0, int bh, int w4,
                                           uint32_t row_bytes, int Nv, int tid)
     {
         // buffer loads: a scalar descriptor at the box origin whose range ends
@@ -363,6 +363,11 @@ struct BoxStage {
         const __amdgpu_buffer_rsrc_t rsrc =
             __builtin_amdgcn_make_buffer_rsrc((void *)base, (short)0, nrec, 0x00020000);
         int off = (int)((uint32_t)(tid >> 4) * row_bytes + (tid & 15) * 4 * ST::BYTES);
+        // lanes past the box's last column (w4: its columns over 4) read zeros outside
+        // the descriptor's range, a quarter of the bytes: 640^2 x 321 FP32 from 120
+        // x 1280 x 900 5.13 -> 5.00 ms, 1024^3 FP16 315 -> 312.  Volumes in shorter
+        // runs sit in the caches, and the test costs them 0.5 to 1 %.
+        if constexpr (TRIM) off = (tid & 15) < w4 ? off : 0x40000000;
         // the packed-FP16 kernel forms the PER offsets anew for every box: held,
         // they would take it past the 96 registers of five waves per SIMD
         if constexpr (ST::PAIRS) asm volatile("" : "+v"(off));
@@ -555,9 +560,10 @@ __global__ void __launch_bounds__(256 * G) bp_kernel(BPArgs<typename Store<S>::R
                     (inner ? 0 : __popcll(mi));
                 if (staged) {
                     // the index with a flag: every tap column lies on the detector
-                    // (columns are below 8192, a box has at most 127 rows)
+                    // (columns are below 8192, a box has at most 127 rows and 63
+                    // columns)
                     const int at = slot * 64 + (lane % G) * (64 / G) + rank;
-                    ebox[at] = make_int4(q.x | q.w << 16, q.y,
+                    ebox[at] = make_int4(q.x | q.w << 16 | ((q.z & 0xff) + 3) / 4 << 24, q.y,
                                          bb | (q.z & BOX_INNER_U ? INNER_U : 0), __float_as_int(c));
                     ess[at] = make_float2(s, a.scales[bb] * wnorm);
                 }
@@ -574,17 +580,18 @@ __global__ void __launch_bounds__(256 * G) bp_kernel(BPArgs<typename Store<S>::R
             angles_of_group(0);
             angles_of_group(1);
             __syncthreads();
-            BoxStage<S, BOX_H> stage;
-            // the box being loaded: first column, first row, last row, index
+            BoxStage<S, BOX_H, (ZR > 16)> stage;
+            // the box being loaded: first column, first row, last row, index (its
+            // columns over 4 in the top byte of the entry)
             int bu0 = 0, bv0 = 0, bh = -1, bi = 0;
             auto issue = [&](const int4 &e) {
                 const int uh = uniform_int(e.x);
                 bu0 = uh & 0xffff;
-                bh = uh >> 16;
+                bh = uh >> 16 & 0xff;
                 bv0 = uniform_int(e.y);
                 bi = uniform_int(e.z);
                 stage.issue(a.stack + (size_t)(bi & ~INNER_U) * a.angle_bytes, bu0, bv0, bh,
-                            a.row_bytes, a.Nv, tid);
+                            uh >> 24, a.row_bytes, a.Nv, tid);
             };
             // column weights and LDS offsets of the staged angle, then its gathers
             auto gather_angle = [&](auto fast_tag, int qu, int qv, bool inner_u, float wc, float ws,
