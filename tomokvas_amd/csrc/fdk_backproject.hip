@@ -50,8 +50,6 @@
 // 1800 x 2048^2):
 //   TKV_BP_ZR_F32 / _F16 / _BF16 / _F16P  slices per thread (register z-run)
 //                                  per storage type (FP64 uses 8)
-//   TKV_BP_LB                      packed FP16: LDS gathers per lane issued
-//                                  together
 //   TKV_BP_BOXP_F32 / _F16P        LDS row pitch of the staged box in 32-bit
 //                                  words (>= 64, multiple of 4): rows of one
 //                                  column fall in different banks (FP32 samples;
@@ -67,9 +65,6 @@
 #endif
 #ifndef TKV_BP_ZR_F16P
 #define TKV_BP_ZR_F16P 32
-#endif
-#ifndef TKV_BP_LB
-#define TKV_BP_LB 4
 #endif
 #ifndef TKV_BP_BOXP_F32
 #define TKV_BP_BOXP_F32 80
@@ -261,62 +256,65 @@ struct LdsGather {
 // along v runs in packed FP16; the two column weights (FP16, normalised to at
 // most U^2) and the two lerped columns meet in one v_dot2_f32_f16, summed in
 // FP32.
-template <bool FAST, int LB, int P>
-__device__ __forceinline__ void gather_pairs(float *acc, const float *az, const float *box,
-                                             float Uv, float cz, const char *col, half2_t wuh,
-                                             float vmax)
-{
-    static_assert(LB % 2 == 0, "fractions are converted in pairs");
-    half2_t c[LB];
-    bool okk[LB];
-#pragma unroll
-    for (int k = 0; k < LB; k += 2) {
-        const float va = fmaf(az[k], Uv, cz), vb = fmaf(az[k + 1], Uv, cz);
+template <bool FAST, int P>
+struct PairGather {
+    half2_t f, w0[2], w1[2];   // the two slices' fractions, their rows iv and iv + 1
+    bool ok[2];
+    __device__ __forceinline__ void issue(const float *az, const float *box, float Uv, float cz,
+                                          const char *col, float vmax)
+    {
+        const float v[2] = {fmaf(az[0], Uv, cz), fmaf(az[1], Uv, cz)};
         // one conversion serves two slices; each lerp broadcasts its half
-        const half2_t fab = __builtin_bit_cast(
-            half2_t, __builtin_amdgcn_cvt_pkrtz(__builtin_amdgcn_fractf(va),
-                                                __builtin_amdgcn_fractf(vb)));
+        f = __builtin_bit_cast(half2_t,
+                               __builtin_amdgcn_cvt_pkrtz(__builtin_amdgcn_fractf(v[0]),
+                                                          __builtin_amdgcn_fractf(v[1])));
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const float v = j ? vb : va;
-            bool ok = true;
             // v >= 0 where used
-            const float *p0 = (const float *)(col + (int)__umul24((unsigned)(int)v, 4u * P));
+            const float *p0 = (const float *)(col + (int)__umul24((unsigned)(int)v[j], 4u * P));
+            ok[j] = true;
             if (!FAST) {
-                ok = v >= 0.f && v <= vmax;
-                p0 = ok ? p0 : box;
+                ok[j] = v[j] >= 0.f && v[j] <= vmax;
+                p0 = ok[j] ? p0 : box;
             }
-            const half2_t w0 = *(const half2_t *)p0;
-            const half2_t w1 = *(const half2_t *)(p0 + P);
-            const half2_t f = j ? half2_t{fab.y, fab.y} : half2_t{fab.x, fab.x};
-            c[k + j] = f * (w1 - w0) + w0;
-            okk[k + j] = ok;
+            w0[j] = *(const half2_t *)p0;
+            w1[j] = *(const half2_t *)(p0 + P);
         }
     }
     // the three-address VOP3P form (the builtin selects the two-address
     // v_dot2c form, whose tied accumulator costs register copies here)
+    __device__ __forceinline__ void add(float *acc, half2_t wuh) const
+    {
 #pragma unroll
-    for (int k = 0; k < LB; ++k) {
-        const half2_t w = okk[k] ? wuh : half2_t{0, 0};
-        float r;
-        asm("v_dot2_f32_f16 %0, %1, %2, %3" : "=v"(r) : "v"(c[k]), "v"(w), "v"(acc[k]));
-        acc[k] = r;
+        for (int j = 0; j < 2; ++j) {
+            const half2_t fj = j ? half2_t{f.y, f.y} : half2_t{f.x, f.x};
+            const half2_t c = fj * (w1[j] - w0[j]) + w0[j];
+            const half2_t w = ok[j] ? wuh : half2_t{0, 0};
+            float r;
+            asm("v_dot2_f32_f16 %0, %1, %2, %3" : "=v"(r) : "v"(c), "v"(w), "v"(acc[j]));
+            acc[j] = r;
+        }
     }
-}
+};
 
 // all ZR slices of a thread for one staged angle
-template <bool FAST, typename ST, int ZR, int LB, int P>
+template <bool FAST, typename ST, int ZR, int P>
 __device__ __forceinline__ void gather_run(float (&acc)[ZR], const float (&az)[ZR],
                                            const float *box, float Uv, float cz,
-                                           const char *col, float wu0, float wu1, half2_t wuh, float vmax,
-                                           float one)
+                                           const char *col, float wu0, float wu1, half2_t wuh,
+                                           float vmax, float one)
 {
     if constexpr (ST::PAIRS && !ST::MIX) {
+        PairGather<FAST, P> g[2];
+        g[0].issue(az, box, Uv, cz, col, vmax);
 #pragma unroll
-        for (int k0 = 0; k0 < ZR; k0 += LB) {
-            gather_pairs<FAST, LB, P>(acc + k0, az + k0, box, Uv, cz, col, wuh, vmax);
+        for (int k = 0; k < ZR; k += 2) {
             __builtin_amdgcn_sched_barrier(0);
+            if (k + 2 < ZR) g[(k / 2 + 1) & 1].issue(az + k + 2, box, Uv, cz, col, vmax);
+            __builtin_amdgcn_sched_barrier(0);
+            g[k / 2 & 1].add(acc + k, wuh);
         }
+        __builtin_amdgcn_sched_barrier(0);
     } else {
         // one slice's samples are on their way while the slice before is added: left
         // to itself the compiler waits for each slice's or holds those of several,
@@ -441,7 +439,7 @@ __device__ __forceinline__ float div_normal(float n, float d)
 // ---- the backprojector --------------------------------------------------------------
 // G: 256-thread groups of a workgroup, each with its own box, that take the
 // staged angles in turn; their sums meet in LDS at the end (see bp_shape)
-template <typename S, int ZR, int LB, int G>
+template <typename S, int ZR, int G>
 __global__ void __launch_bounds__(256 * G) bp_kernel(BPArgs<typename Store<S>::R> a)
 {
     using R = typename Store<S>::R;
@@ -628,7 +626,7 @@ __global__ void __launch_bounds__(256 * G) bp_kernel(BPArgs<typename Store<S>::R
                 if constexpr (PACKED) wuh = half2_t{(_Float16)wu0, (_Float16)wu1};
                 // sample (row iv, column iu) lies at col + iv*4*P
                 const char *col = (const char *)boxmem + (iu * 4 - (qu * 4 + qv * (4 * P)));
-                gather_run<FAST, ST, ZR, LB, P>(acc, az, boxmem, Uv, cz, col, wu0, wu1, wuh,
+                gather_run<FAST, ST, ZR, P>(acc, az, boxmem, Uv, cz, col, wu0, wu1, wuh,
                                                 a.vmax, a.one);
             };
             using fast_t = std::integral_constant<bool, true>;
@@ -883,13 +881,12 @@ static int launch_bp_z(const BPLaunch &L, hipStream_t st)
     if (!grid_fits(nb, 256)) return fail(FDK_ERR_UNSUPPORTED, "backproject: volume too large");
     a.nblocks = (int)nb;
     a.box_h = Store<S>::STAGED ? box_height<ZR>(L) : 0;
-    constexpr int LB = ZR < TKV_BP_LB ? ZR : TKV_BP_LB;
     const size_t lds = sizeof(float) * Store<S>::P * a.box_h * G;
     // beyond 64 KiB a workgroup takes up to the 160 KiB of LDS of a gfx950 CU
     if (lds > 61440)
-        TKV_HIP(hipFuncSetAttribute((const void *)bp_kernel<S, ZR, LB, G>,
+        TKV_HIP(hipFuncSetAttribute((const void *)bp_kernel<S, ZR, G>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((bp_kernel<S, ZR, LB, G>), dim3((unsigned)nb), dim3(256 * G), lds, st, a);
+    hipLaunchKernelGGL((bp_kernel<S, ZR, G>), dim3((unsigned)nb), dim3(256 * G), lds, st, a);
     TKV_HIP(hipGetLastError());
     return FDK_OK;
 }
