@@ -383,6 +383,12 @@ int filter_and_pack(fdk_ctx *c, const float *in, float *filt, int nang, unsigned
                             maxabs, c->storage, stack, scales, st);
 }
 
+// largest |z| that a z-run may hold, the table's padding included
+double table_reach(const fdk_ctx *c)
+{
+    return c->g.scale * (0.5 * c->g.Nz + std::fabs((double)c->g.cz) + 64.);
+}
+
 // Slices [z0, z0 + nz) of the volume into vol (nz < 0: every slice).
 int stage_backproject(fdk_ctx *c, int store_dtype, const void *stack, const void *scales,
                       int ang0, int nang, void *vol, int accumulate, hipStream_t st,
@@ -412,7 +418,7 @@ int stage_backproject(fdk_ctx *c, int store_dtype, const void *stack, const void
     L.out_scale = out_scale(c, store_dtype);
     L.maskR2 = 0.25 * (double)c->g.Nu * (double)c->g.Nu;
     L.scale = c->g.scale;
-    L.az_max = L.scale * (0.5 * c->g.Nz + std::fabs((double)c->g.cz) + 64.);   // with z padding
+    L.az_max = table_reach(c);
     L.accumulate = accumulate;
     // from the whole volume, so that a volume in z-chunks gets the same sums
     L.shape = tkv::bp_shape(store_dtype, c->g.Nx, c->g.Ny, c->g.Nz);
@@ -1276,30 +1282,39 @@ int fdk_forward_project(fdk_ctx *c, int dtype, const void *d_vol, int ang0, int 
     L.D = c->g.D;
     L.out_scale = out_scale(c, dtype);
     L.maskR2 = 0.25 * (double)c->g.Nu * (double)c->g.Nu;
+    L.scale = c->g.scale;
+    L.az_max = table_reach(c);
     {
         // A voxel adds at most U^2 |x| hat(u - col) hat(v - row), hat(t) =
-        // max(0, 1 - |t|), to a detector sample; U is bounded per tile by the
-        // kernel (the staged path never sees U >= 100: its footprints need
-        // D-S > D/100).  The hats of a 32 x 32-column, 64-slice workgroup sum to
-        // at most 32 S(du) S(dv), S(d) the largest sum of hats at points d or
-        // more apart (the sum is piecewise linear in a shift of the points, and
-        // bends downwards only where a point meets a peak):
+        // max(0, 1 - |t|), to a detector sample; U < D/(D - r) (and the staged path
+        // never sees U >= 100: its footprints need D-S > D/100).  The hats of n x n
+        // columns x 64 slices sum to at most n S(du) S(dv), S(d) the largest sum of
+        // hats at points d or more apart (the sum is piecewise linear in a shift of the
+        // points, and bends downwards only where a point meets a peak); N(d) of these
+        // points lie under one hat:
         //  - along z the rows v of a column are scale * U >= scale*D/(D+r) apart;
-        //  - along each of the 32 lines of the tile axis closer to the T
+        //  - along each of the n lines of the tile axis closer to the T
         //    direction (|cos| or |sin| >= 1/sqrt 2), u = cX + D T/(D-S) is
         //    monotone with |du/d(step)| = pitch D |c'(D-S) + T s'| / (D-S)^2 >=
         //    pitch D (D - 2r) / (sqrt 2 (D+r)^2) (|S|, |T| < r; no bound, so
-        //    32 hats of 1, if D <= 2r).
+        //    n hats of 1, if D <= 2r).
         const double r = std::sqrt(L.maskR2), D = c->g.D;
-        const double pitch = std::fabs((double)c->g.scale);
+        const double pitch = L.scale;
         auto hats = [](double d, double most) {
             const double m = d > 0.0 ? std::floor(1.0 / d) : most;
             return m >= most ? most : std::min(most, 1.0 + 2.0 * m - d * m * (m + 1.0));
         };
+        auto count = [](double d, double most) {
+            return d > 0.0 ? std::min(most, 1.0 + std::floor(2.0 / d)) : most;
+        };
         const double du = D > 2.0 * r
                               ? pitch * D * (D - 2.0 * r) / (std::sqrt(2.0) * (D + r) * (D + r))
                               : 0.0;
-        L.fx_bound = 32.0 * hats(du, 32.0) * hats(pitch * D / (D + r), 64.0);
+        const double dv = pitch * D / (D + r);
+        L.umax_cyl = D > r ? std::min(100.0, D / (D - r)) : 100.0;
+        L.fx_tile = 32.0 * hats(du, 32.0) * hats(dv, 64.0);
+        L.fx_block = 16.0 * hats(du, 16.0) * hats(dv, 64.0);
+        L.fx_count = 16.0 * count(du, 16.0) * count(dv, 64.0) * L.umax_cyl * L.umax_cyl;
     }
     return tkv::launch_forward_project(f64 ? 8 : 4, L, pick(c, stream));
 }

@@ -139,10 +139,12 @@ struct FPLaunch {           // adjoint of the backprojector
     int Nu, Nv, nang;
     int Nx, Ny, Nz;
     double cX, cZ, D, out_scale, maskR2;
-    // FP32 path: bound on the sum of the bilinear weights with which a workgroup's
-    // voxels splat onto one detector sample (it fixes the scale of its
-    // fixed-point accumulation)
-    double fx_bound;
+    double scale, az_max;   // voxel pitch, largest |z| of a z-run
+    // FP32 path, for the scale of its fixed-point sums.  Bounds, for U = 1, on the sum
+    // of the bilinear weights with which the voxels of 32 x 32 columns x 64 slices, and
+    // of 16 x 16 x 64, splat onto one detector sample; the number of voxels of 16 x 16
+    // x 64 that reach one, times the largest U^2; the largest U
+    double fx_tile, fx_block, fx_count, umax_cyl;
 };
 int launch_forward_project(int real_bytes, const FPLaunch &a, hipStream_t st);
 
