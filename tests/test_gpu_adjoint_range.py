@@ -1,5 +1,5 @@
-"""The FP32 adjoint on volumes whose voxels differ widely in size, against the same splats
-summed in double."""
+"""The FP32 adjoint on volumes whose voxels differ widely in size, and on voxels
+that are not finite, against the same splats summed in double."""
 import numpy as np
 import pytest
 
@@ -118,3 +118,31 @@ def test_a_large_voxel_sets_the_step_of_its_own_columns(torch, case, at, ratio):
     err = O.rel_rmse(got[far], ref[far])
     say(f"  error of the samples out of its block's reach {err:.2e}")
     assert far.any() and err <= 1e-6
+
+
+# 32-bit sums at every angle, and 64-bit ones at every angle
+ODD = {"narrow": NARROW["one"], "wide": WIDE["two"][0]}
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf, 3e38])
+@pytest.mark.parametrize("case", list(ODD))
+def test_voxels_that_are_not_finite_reach_their_samples(torch, case, value):
+    """Such a voxel, or one whose sums overflow fixed point, makes the samples that it
+    reaches not finite (or large) and changes no others."""
+    g = scan(**ODD[case], tau=0.1)
+    x = np.random.default_rng(9).standard_normal((g.Nz, g.Ny, g.Nx)).astype(f32)
+    x[20, 25, 23] = x[33, 40, 12] = 0
+    say(f"voxels that are not finite {case}, {value}")
+    odd = np.zeros_like(x)
+    odd[20, 25, 23] = odd[33, 40, 12] = 1
+    ref, hit = splats(g, x), splats(g, odd)
+    x[odd == 1] = value
+    got = project(torch, g, x)
+    assert np.count_nonzero(hit) >= 2 * 4 * g.Nang - 8
+    # a weight of a few FP32 roundings of zero may be zero there
+    reached = hit > 1e-5 * hit.max()
+    if np.isfinite(value):
+        assert O.rel_rmse(got[reached], (hit * value)[reached]) <= 5e-7
+    else:
+        assert not np.isfinite(got[reached]).any()
+    assert O.rel_rmse(got[hit == 0], ref[hit == 0]) <= 1e-6

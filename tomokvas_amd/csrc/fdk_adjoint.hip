@@ -220,9 +220,9 @@ __device__ inline bool narrow_angle(const FPArgs<float> &a, float c, float s, in
 // 2^-K with K about 49 of a tile whose largest voxel is scaled to [1/2, 1): within
 // 2^-26 of the voxel's weight down to 2^(25 - K) of the largest voxel, with exact sums.
 //
-// Voxels that 64-bit sums can't hold -- infinities, NaN, and the relatively smallest --
-// are splatted straight into HBM in a pass of their own, and so are the angles whose
-// footprint is beyond the box.
+// Voxels that fixed point can't hold -- infinities, NaN, and the largest (32 bits) or
+// the relatively smallest (64 bits) -- are splatted straight into HBM in a pass of
+// their own, and so are the angles whose footprint is beyond the box.
 //
 // What bounds it: a splat costs 22 vector instructions (about 1.1 issue cycles
 // of the CU each; plain FP32 and integer adds and multiplies 0.75) beside 16
@@ -333,7 +333,8 @@ __global__ void __launch_bounds__(FP_THREADS) fp_lds_kernel(FPArgs<float> a)
     // the barriers below are workgroup-wide: skip only whole workgroups
     if (!__syncthreads_or(live != 0)) return;
 
-    // the largest |voxel| of each block, of those that 64-bit sums can hold
+    // the largest |voxel| of each block, of those that fixed point can hold
+    constexpr float TOP = WIDE ? __builtin_inff() : 0x1p100f;
     bool odd = false;
     {
         float m[NB];
@@ -342,7 +343,7 @@ __global__ void __launch_bounds__(FP_THREADS) fp_lds_kernel(FPArgs<float> a)
 #pragma unroll
         for (int j = 0; j < NC; ++j) {
             const float g = fabsf(val[j]);
-            const bool fits = !WIDE || g < __builtin_inff();
+            const bool fits = g < TOP;
             odd = odd || !fits;
             m[block_of(j)] = fmaxf(m[block_of(j)], fits ? g : 0.f);
         }
@@ -389,9 +390,7 @@ __global__ void __launch_bounds__(FP_THREADS) fp_lds_kernel(FPArgs<float> a)
     }
     // beyond this magnification K would leave too few bits
     const bool steep = WIDE && umax > 4.f;
-    auto straight = [&](float g) {
-        return WIDE && g != 0.f && !(fabsf(g) >= least && fabsf(g) < __builtin_inff());
-    };
+    auto straight = [&](float g) { return g != 0.f && !(fabsf(g) >= least && fabsf(g) < TOP); };
     // only voxels for fixed point are left
     auto settle = [&]() {
 #pragma unroll
