@@ -1,0 +1,45 @@
+"""Calls at the edges of what the entry points accept, each against the oracle or the
+general path."""
+import numpy as np
+import pytest
+
+import oracle as O
+from tomokvas_amd import _lib
+
+from gpu_util import ogeom, say, scan, stages
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch():
+    import torch as t
+    assert t.cuda.is_available(), "GPU tests need a HIP device"
+    return t
+
+
+def decoded(torch, st, g, stack, scales, store):
+    """The stored samples as float [Nv][Nang][Nu] on the host."""
+    dt = {_lib.F32: torch.float32, _lib.F16: torch.float16, _lib.F16_PACKED: torch.float16,
+          _lib.BF16: torch.bfloat16}[store]
+    per = st.stack_bytes(store, 1) - st.stack_bytes(store, 0)
+    q = stack[:per * g.Nang].view(dt).view(g.Nang, g.Nv, -1)[:, :, :g.Nu].float()
+    return (q * scales[:, None, None]).transpose(0, 1).contiguous().cpu().numpy()
+
+
+# the reciprocal of D - S leaves the normal numbers beyond 2^126
+@pytest.mark.parametrize("D", [1e30, 8.6e37, 3.4e38])
+@pytest.mark.parametrize("store", [_lib.F32, _lib.F16, _lib.BF16, _lib.F16_PACKED])
+def test_backprojection_of_a_parallel_beam(torch, D, store):
+    """A source so far away that U = 1 for every voxel."""
+    g = scan(60, 40, 9, 40, 37, 33, D=D, tau=0.1)
+    st = stages(g)
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    d = torch.randn(st.sino_shape(), device="cuda", generator=gen)
+    say(f"parallel beam D {D:g}, storage {store}")
+    stack, scales = st.pack(d, store, d.abs().amax(dim=(0, 2)).view(torch.int32))
+    got = st.backproject(stack, store, scales).cpu().numpy()
+    ref = O.backproject(ogeom(g), decoded(torch, st, g, stack, scales, store))
+    assert np.abs(ref).max() > 0
+    # FP32 sums in another order; packed FP16 also rounds weights and lerps to FP16
+    assert O.rel_rmse(got, ref) <= (1e-3 if store == _lib.F16_PACKED else 1e-6)

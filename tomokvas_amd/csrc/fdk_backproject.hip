@@ -426,7 +426,8 @@ __device__ __forceinline__ float uniform_load(const float *p)
 // n / d correctly rounded (Markstein 1990: a Newton step on the reciprocal, two
 // residual corrections of the quotient) for normal n, d and quotient: without
 // the exponent scaling and special cases of the general division, 9
-// instructions instead of 13.  The staged angles have d = D - S > D/100.
+// instructions instead of 13.  The staged angles have d = D - S > D/100, and D is
+// at least 1/2 and at most 2^100 here.
 __device__ __forceinline__ float div_normal(float n, float d)
 {
     float r = __builtin_amdgcn_rcpf(d);
@@ -866,7 +867,10 @@ static int launch_bp_z(const BPLaunch &L, hipStream_t st)
     a.nang = L.nang;
     a.cX = (R)L.cX;
     a.cZ = (R)L.cZ;
-    a.D = (R)L.D;
+    // FP32: from 2^100 on D - S rounds to D and U is 1 (|S| < 4096 in the cylinder),
+    // and the reciprocal in div_normal stays a normal number
+    const bool far = sizeof(R) == 4 && L.D > 0x1p100 && std::isfinite((R)L.D);
+    a.D = far ? (R)0x1p100 : (R)L.D;
     a.umax = (R)(L.Nu - 1);
     a.vmax = (R)(L.Nv - 1);
     a.out_scale = (R)L.out_scale;
