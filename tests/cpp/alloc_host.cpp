@@ -1,0 +1,122 @@
+// The engine's handling of allocations that fail, on the CPU: this program defines
+// the HIP calls the library makes (memory from malloc, kernels only counted), so that
+// an allocation can be refused when the test says so.  `alloc_host MODE` prints one
+// line per checked fact and returns 0 if all hold.
+#include "tomokvas/fdk.h"
+
+#include <hip/hip_runtime_api.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <string>
+#include <utility>
+#include <vector>
+
+namespace {
+int launches = 0, allowed = -1, device = 0;   // allocations left (-1: any number)
+std::map<void *, std::pair<size_t, int>> live;   // bytes and device of each allocation
+}
+
+extern "C" {
+hipError_t hipGetDeviceCount(int *n) { *n = 2; return hipSuccess; }
+hipError_t hipSetDevice(int d) { device = d; return hipSuccess; }
+hipError_t hipGetDevice(int *d) { *d = device; return hipSuccess; }
+hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipMalloc(void **p, size_t n)
+{
+    if (allowed == 0) return hipErrorOutOfMemory;
+    if (allowed > 0) --allowed;
+    *p = std::calloc(1, n);
+    live[*p] = {n, device};
+    return hipSuccess;
+}
+hipError_t hipFree(void *p)
+{
+    live.erase(p);
+    std::free(p);
+    return hipSuccess;
+}
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind)
+{
+    std::memcpy(d, s, n);
+    return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *, const void *, size_t, hipMemcpyKind, hipStream_t) { return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = (hipStream_t)&launches; return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t *e) { *e = (hipEvent_t)&launches; return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCreate(e); }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { *ms = 0; return hipSuccess; }
+hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
+hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *) { return hipSuccess; }
+hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t)
+{
+    ++launches;
+    return hipSuccess;
+}
+}
+
+namespace {
+bool good = true;
+void check(const char *what, bool ok)
+{
+    std::printf("%s: %s\n", ok ? "ok" : "FAILED", what);
+    if (!ok) good = false;
+}
+
+fdk_ctx *context(int gpu, int storage)
+{
+    fdk_ctx *c = nullptr;
+    std::vector<float> sino(40 * 12 * 30, 1.f);
+    if (fdk_create(gpu, &c) || fdk_set_sinogram_properties(c, sino.data(), 40, 19.5f, 12, 30, 14.5f, 0.5f, 200.f, 0.1f) ||
+        fdk_set_reconstruction_properties(c, 24, 11.5f, 24, 11.5f, 16, 7.5f, 0.f) ||
+        fdk_set_storage(c, storage) || fdk_initialize(c)) {
+        std::printf("FAILED: %s\n", fdk_last_error_string());
+        std::exit(1);
+    }
+    return c;
+}
+}
+
+int main(int argc, char **argv)
+{
+    const std::string mode = argc > 1 ? argv[1] : "";
+    if (mode == "stack") {
+        // a larger stored stack can't be had: no reconstruction runs without one
+        fdk_ctx *c = context(0, FDK_BF16);
+        allowed = 0;
+        check("storage refused", fdk_set_storage(c, FDK_F32) == FDK_ERR_OUT_OF_MEMORY);
+        launches = 0;
+        check("not initialized", fdk_calculate_reconstruction(c, nullptr, nullptr) == FDK_ERR_NOT_INITIALIZED);
+        check("no launch", launches == 0);
+        check("no projections", fdk_device_sinogram(c) == nullptr);
+        allowed = -1;
+        check("initialized again", fdk_initialize(c) == FDK_OK);
+        check("reconstruction", fdk_calculate_reconstruction(c, nullptr, nullptr) == FDK_OK && launches > 0);
+        fdk_destroy(c);
+    } else if (mode == "filtered") {
+        // the stack fits, the filtered projections don't: the old storage goes on
+        fdk_ctx *c = context(0, FDK_F32);
+        allowed = 0;
+        check("storage refused", fdk_set_storage(c, FDK_F16) == FDK_ERR_OUT_OF_MEMORY);
+        check("reconstruction in F32", fdk_calculate_reconstruction(c, nullptr, nullptr) == FDK_OK);
+        allowed = -1;
+        check("storage accepted", fdk_set_storage(c, FDK_F16) == FDK_OK);
+        check("reconstruction in F16", fdk_calculate_reconstruction(c, nullptr, nullptr) == FDK_OK);
+        fdk_destroy(c);
+    } else {
+        std::printf("FAILED: unknown mode\n");
+        return 2;
+    }
+    check("nothing left allocated", live.empty());
+    return good ? 0 : 1;
+}

@@ -891,7 +891,11 @@ int fdk_set_storage(fdk_ctx *c, int dtype)
         if (!rc && scaled_storage(dtype))
             rc = ensure((void **)&c->d_filt, c->cap_filt,
                         (size_t)c->g.Nu * c->g.Nv * c->g.Nang * sizeof(float), "filtered stack");
-        if (rc) return rc;
+        if (rc) {
+            // the old storage goes on if its stack is still there
+            if (!c->d_stack) c->initialized = false;
+            return rc;
+        }
     }
     c->storage = dtype;
     return FDK_OK;
