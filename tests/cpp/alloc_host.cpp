@@ -113,6 +113,15 @@ int main(int argc, char **argv)
         check("storage accepted", fdk_set_storage(c, FDK_F16) == FDK_OK);
         check("reconstruction in F16", fdk_calculate_reconstruction(c, nullptr, nullptr) == FDK_OK);
         fdk_destroy(c);
+    } else if (mode == "device") {
+        // another device is current when the storage grows
+        fdk_ctx *c = context(1, FDK_BF16);
+        (void)hipSetDevice(0);
+        check("storage accepted", fdk_set_storage(c, FDK_F32) == FDK_OK);
+        bool own = true;
+        for (const auto &a : live) own = own && a.second.second == 1;
+        check("every allocation on the context's device", own);
+        fdk_destroy(c);
     } else {
         std::printf("FAILED: unknown mode\n");
         return 2;

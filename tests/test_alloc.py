@@ -28,3 +28,8 @@ def exe(tmp_path_factory):
 def test_storage_that_cannot_be_allocated(exe, mode):
     r = subprocess.run([exe, mode], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr[-2000:]
+
+
+def test_storage_grows_on_the_context_s_device(exe):
+    r = subprocess.run([exe, "device"], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr[-2000:]

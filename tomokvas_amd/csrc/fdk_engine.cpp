@@ -886,8 +886,10 @@ int fdk_set_storage(fdk_ctx *c, int dtype)
     if (dtype != FDK_F32 && dtype != FDK_F16 && dtype != FDK_BF16 && dtype != FDK_F16_PACKED)
         return fail(FDK_ERR_INVALID_ARGUMENT, "storage must be F32, F16, BF16 or F16_PACKED");
     if (c->initialized && dtype != c->storage) {
-        int rc = ensure(&c->d_stack, c->cap_stack, fdk_stack_bytes(c, dtype, c->g.Nang),
-                        "stored stack");
+        int rc = set_device(c);
+        if (rc) return rc;
+        rc = ensure(&c->d_stack, c->cap_stack, fdk_stack_bytes(c, dtype, c->g.Nang),
+                    "stored stack");
         if (!rc && scaled_storage(dtype))
             rc = ensure((void **)&c->d_filt, c->cap_filt,
                         (size_t)c->g.Nu * c->g.Nv * c->g.Nang * sizeof(float), "filtered stack");
