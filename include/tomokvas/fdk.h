@@ -174,7 +174,8 @@ size_t fdk_stack_bytes(fdk_ctx *ctx, int store_dtype, int nang);
 /* fdk_filter out of place, for nang projections from the angle that d_in points at of
  * a stack [Nv][in_nang][Nu].  store_dtype < 0: rows [Nv][nang][Nu] into d_out, with
  * weight 0, 1 (before the filter, W then F_h) or 2 (after it; with `adjoint` the
- * transpose W F_h^T); d_out may be d_in when nang = in_nang.  store_dtype F32 or BF16
+ * transpose W F_h^T); d_out may be d_in when nang = in_nang, and meets none of the
+ * rows read otherwise (refused).  store_dtype F32 or BF16
  * (F32 data) or F64: weighted and filtered into the stored stack and scales that
  * fdk_pack would write (weight 1, no adjoint, no d_maxabs). */
 int fdk_filter_into(fdk_ctx *ctx, int dtype, const void *d_in, int in_nang, int nang,

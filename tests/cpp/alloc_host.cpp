@@ -1,11 +1,12 @@
-// The engine's handling of allocations that fail, on the CPU: this program defines
-// the HIP calls the library makes (memory from malloc, kernels only counted), so that
-// an allocation can be refused when the test says so.  `alloc_host MODE` prints one
-// line per checked fact and returns 0 if all hold.
+// The engine's host code on the CPU: this program defines the HIP calls the library
+// makes (memory from malloc, kernels only counted), so that an allocation can be
+// refused when the test says so, and a call be seen to launch nothing.  `alloc_host
+// MODE` prints one line per checked fact and returns 0 if all hold.
 #include "tomokvas/fdk.h"
 
 #include <hip/hip_runtime_api.h>
 
+#include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -121,6 +122,46 @@ int main(int argc, char **argv)
         bool own = true;
         for (const auto &a : live) own = own && a.second.second == 1;
         check("every allocation on the context's device", own);
+        fdk_destroy(c);
+    } else if (mode == "overlap") {
+        // fdk_filter_into: rows [Nv][nang][Nu] = [30][12][40] and stored stacks
+        fdk_ctx *c = context(0, FDK_F32);
+        const size_t n = 40 * 12 * 30;
+        std::vector<float> buf(4 * n + fdk_stack_bytes(c, FDK_F32, 12) / 4 + 8);
+        float *p = buf.data();
+        while ((uintptr_t)p & 15) ++p;
+        float scales[12];
+        auto into = [&](const float *in, int in_nang, int nang, int store, void *out) {
+            launches = 0;
+            const int rc = fdk_filter_into(c, FDK_F32, in, in_nang, nang, store < 0 ? 0 : 1, 0, store, out,
+                                           store < 0 ? nullptr : scales, nullptr, nullptr);
+            return rc == FDK_OK && launches > 0 ? 1 : rc == FDK_ERR_INVALID_ARGUMENT && launches == 0 ? 0 : -1;
+        };
+        check("in place", into(p, 12, 12, -1, p) == 1);
+        check("out of place, side by side", into(p, 12, 12, -1, p + n) == 1 && into(p + n, 12, 12, -1, p) == 1);
+        check("one row further", into(p, 12, 12, -1, p + 40) == 0);
+        check("one row before", into(p + 40, 12, 12, -1, p) == 0);
+        check("the last sample", into(p, 12, 12, -1, p + n - 1) == 0 && into(p + n - 1, 12, 12, -1, p) == 0);
+        // angles [4, 9) of 12: from row 4 of the first detector row to row 8 of the last
+        const float *s = p + 4 * 40;
+        check("a slice", into(s, 12, 5, -1, p + n) == 1);
+        check("a slice onto its first sample", into(s, 12, 5, -1, (void *)s) == 0);
+        check("a slice onto the gap before it", into(p + n, 12, 5, -1, p + n - 5 * 40 * 30) == 1);
+        check("a slice onto its last sample", into(s, 12, 5, -1, p + n - 3 * 40 - 1) == 0);
+        check("after a slice's last sample", into(s, 12, 5, -1, p + n - 3 * 40) == 1);
+        // one angle of 45 in a stack of 30 x 45 rows; its 30 rows fit between two of its rows
+        check("between a slice's rows", into(p, 45, 1, -1, p + 40) == 1 && into(p, 45, 1, -1, p + 15 * 40) == 1 &&
+                                            into(p, 45, 1, -1, p + 15 * 40 + 1) == 0 &&
+                                            into(p, 45, 1, -1, p + 39) == 0 &&
+                                            into(p, 45, 1, -1, p + 3 * 45 * 40 + 40) == 1 &&
+                                            into(p, 45, 1, -1, p + 29 * 45 * 40 + 39) == 0 &&
+                                            into(p, 45, 1, -1, p + 29 * 45 * 40 + 40) == 1);
+        check("into a stack", into(p, 12, 12, FDK_F32, p + n) == 1 && into(p, 12, 12, FDK_BF16, p + n) == 1);
+        check("into a stack over the rows", into(p, 12, 12, FDK_F32, p) == 0 && into(p + 8, 12, 12, FDK_BF16, p) == 0);
+        const size_t rows = fdk_stack_bytes(c, FDK_BF16, 12) - fdk_stack_bytes(c, FDK_BF16, 0);
+        check("rows right after a stack", into(p + rows / 4, 12, 12, FDK_BF16, p) == 1 &&
+                                              into(p + rows / 4 - 1, 12, 12, FDK_BF16, p) == 0);
+        check("no angles", fdk_filter_into(c, FDK_F32, p, 12, 0, 0, 0, -1, p + 1, nullptr, nullptr, nullptr) == FDK_OK);
         fdk_destroy(c);
     } else {
         std::printf("FAILED: unknown mode\n");

@@ -1,5 +1,5 @@
-"""The engine when an allocation fails, on the CPU: tests/cpp/alloc_host.cpp defines the
-HIP calls that the library makes and refuses memory where the test wants it."""
+"""The engine's host code on the CPU: tests/cpp/alloc_host.cpp defines the HIP calls that
+the library makes, refuses memory where the test wants it and counts launches."""
 import os
 import subprocess
 
@@ -32,4 +32,9 @@ def test_storage_that_cannot_be_allocated(exe, mode):
 
 def test_storage_grows_on_the_context_s_device(exe):
     r = subprocess.run([exe, "device"], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr[-2000:]
+
+
+def test_filter_into_overlapping_buffers(exe):
+    r = subprocess.run([exe, "overlap"], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr[-2000:]

@@ -1191,6 +1191,18 @@ int fdk_filter(fdk_ctx *c, int dtype, void *d_sino, int nang, int weight, int ad
                         pick(c, stream));
 }
 
+// Whether [out, out + bytes) meets a row of the nang projections at in, of a stack
+// [Nv][in_nang][Nu] of rb-byte samples
+static bool meets_rows(const tkv::Geometry &g, const void *in, int in_nang, int nang, size_t rb,
+                       const void *out, size_t bytes)
+{
+    const long long row = (long long)rb * g.Nu, period = row * in_nang, len = row * nang;
+    const long long o0 = (long long)((intptr_t)out - (intptr_t)in), o1 = o0 + (long long)bytes;
+    if (len == 0) return false;
+    const long long v = o0 < len ? 0 : (o0 - len) / period + 1;   // first that ends after o0
+    return v < g.Nv && v * period < o1;
+}
+
 int fdk_filter_into(fdk_ctx *c, int dtype, const void *d_in, int in_nang, int nang, int weight,
                     int adjoint, int store_dtype, void *d_out, void *d_scales,
                     uint32_t *d_maxabs, void *stream)
@@ -1204,9 +1216,13 @@ int fdk_filter_into(fdk_ctx *c, int dtype, const void *d_in, int in_nang, int na
     if (weight < 0 || weight > 2)
         return fail(FDK_ERR_INVALID_ARGUMENT, "filter_into: weight is 0, 1 or 2");
     if (!d_in || !d_out) return fail(FDK_ERR_INVALID_ARGUMENT, "filter_into: null buffer");
+    const size_t rb = dtype == FDK_F64 ? 8 : 4;
     if (store_dtype < 0) {
         if (d_in == d_out && in_nang != nang)
             return fail(FDK_ERR_INVALID_ARGUMENT, "filter_into: in place needs all the angles");
+        if (d_in != d_out &&
+            meets_rows(c->g, d_in, in_nang, nang, rb, d_out, rb * c->g.Nu * c->g.Nv * nang))
+            return fail(FDK_ERR_INVALID_ARGUMENT, "filter_into: output over the input");
         return tkv::launch_filter(
             dtype == FDK_F64 ? 8 : 4,
             filter_launch(c, dtype, d_in, in_nang, d_out, nang, weight, adjoint, d_maxabs),
@@ -1218,6 +1234,9 @@ int fdk_filter_into(fdk_ctx *c, int dtype, const void *d_in, int in_nang, int na
         return fail(FDK_ERR_INVALID_ARGUMENT, "filter_into: a stored stack is W then F_h");
     if ((uintptr_t)d_out & 15)
         return fail(FDK_ERR_INVALID_ARGUMENT, "filter_into: stored stack not 16-byte aligned");
+    if (meets_rows(c->g, d_in, in_nang, nang, rb, d_out,
+                   sample_bytes(store_dtype) * (size_t)tkv::stack_pitch(c->g.Nu) * c->g.Nv * nang))
+        return fail(FDK_ERR_INVALID_ARGUMENT, "filter_into: stored stack over the input");
     return stage_filter_store(c, store_dtype, d_in, in_nang, nang, d_out, d_scales,
                               pick(c, stream));
 }
