@@ -43,3 +43,25 @@ def test_backprojection_of_a_parallel_beam(torch, D, store):
     assert np.abs(ref).max() > 0
     # FP32 sums in another order; packed FP16 also rounds weights and lerps to FP16
     assert O.rel_rmse(got, ref) <= (1e-3 if store == _lib.F16_PACKED else 1e-6)
+
+
+def test_stored_stacks_that_do_not_fit_are_refused(torch):
+    """A stack or scales that are strided, on the host, too small or of another type."""
+    g = scan(40, 12, 9, 16, 16, 16, D=200.0, tau=0.1)
+    st = stages(g)
+    d = torch.randn(st.sino_shape(), device="cuda")
+    for store in (_lib.F32, _lib.BF16):
+        stack, scales = st.pack(d, store)
+        n = stack.numel()
+        bad = [(stack.cpu(), scales), (stack, scales.cpu()), (stack[:n - 1], scales),
+               (torch.zeros(2 * n, dtype=torch.uint8, device="cuda")[::2], scales),
+               (stack, scales[:-1]), (stack, scales.double()), (stack, scales.half()),
+               (stack, torch.zeros(2 * g.Nang, device="cuda")[::2])]
+        for a, b in bad:
+            with pytest.raises(ValueError):
+                st.filter_store(d, store, a, b)
+            with pytest.raises(ValueError):
+                st.pack_into(d, store, a, b, 0)
+        st.filter_store(d, store, stack, scales)
+        st.pack_into(d, store, stack, scales, 0)
+        torch.cuda.synchronize()

@@ -94,10 +94,9 @@ class Stages:
         [ang0, ang0 + n) of a stored stack (F32 or BF16 for F32 data, or F64)."""
         _check_dev(sino)
         n = sino.shape[1] - src0 if n is None else n
-        per = self.stack_bytes(store_dtype, 1) - self.stack_bytes(store_dtype, 0)
-        if min(ang0, src0, n) < 0 or ang0 + n > scales.numel() or src0 + n > sino.shape[1] or \
-                tuple(sino.shape) != self.sino_shape(sino.shape[1]) or \
-                stack.numel() < self.stack_bytes(store_dtype, ang0 + n):
+        per = self._check_stack("filter_store", sino, store_dtype, stack, scales, ang0, n)
+        if min(src0, n) < 0 or src0 + n > sino.shape[1] or \
+                tuple(sino.shape) != self.sino_shape(sino.shape[1]):
             raise ValueError("filter_store: projections outside the stack")
         self._filter_into(sino, src0, n, 1, False, store_dtype, stack.data_ptr() + ang0 * per,
                           scales.data_ptr() + ang0 * scales.element_size(), None)
@@ -111,6 +110,18 @@ class Stages:
     def stack_bytes(self, store_dtype, nang=None):
         return self.L.fdk_stack_bytes(self.fbp.handle, store_dtype,
                                       self.Nang if nang is None else nang)
+
+    def _check_stack(self, what, sino, store_dtype, stack, scales, ang0, n):
+        """Projections [ang0, ang0 + n) lie in the stored stack and its scales (of the
+        data's type: F64 data is stored as F64 only); returns the bytes of one."""
+        _check_dev(stack)
+        _check_dev(scales)
+        if scales.dtype != sino.dtype:
+            raise ValueError(f"{what}: scales of another type")
+        if ang0 < 0 or ang0 + n > scales.numel() or \
+                stack.numel() * stack.element_size() < self.stack_bytes(store_dtype, ang0 + n):
+            raise ValueError(f"{what}: projections outside the stack")
+        return self.stack_bytes(store_dtype, 1) - self.stack_bytes(store_dtype, 0)
 
     def pack(self, filtered, store_dtype, maxabs=None):
         """Returns (stored stack as a uint8 tensor, scales tensor)."""
@@ -132,10 +143,7 @@ class Stages:
         stored stack of stack_bytes(store_dtype) bytes and its scales."""
         _check_dev(filtered)
         n = filtered.shape[1]
-        per = self.stack_bytes(store_dtype, 1) - self.stack_bytes(store_dtype, 0)
-        if ang0 < 0 or ang0 + n > scales.numel() or \
-                stack.numel() < self.stack_bytes(store_dtype, ang0 + n):
-            raise ValueError("pack_into: projections outside the stack")
+        per = self._check_stack("pack_into", filtered, store_dtype, stack, scales, ang0, n)
         mp = maxabs.data_ptr() if maxabs is not None else None
         _lib.check(self.L.fdk_pack(self.fbp.handle, _dtype_code(filtered), filtered.data_ptr(),
                                    n, mp, store_dtype, stack.data_ptr() + ang0 * per,
