@@ -54,7 +54,8 @@ def ramlak_taps(st: Stages) -> np.ndarray:
 
 def _slice(x, a0, n):
     """Projections [a0, a0 + n) of a stack that is not contiguous, as a copy."""
-    return x[:, a0:a0 + n, :].contiguous() if n < x.shape[1] else x.detach().clone()
+    # (clone() would keep the strides of a transposed view)
+    return x[:, a0:a0 + n, :].detach().contiguous()
 
 
 def forward(st: Stages, proj, storage=_lib.F32, chunk=None):
