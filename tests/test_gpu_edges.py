@@ -91,3 +91,28 @@ def test_projections_that_are_not_contiguous(torch, store, chunk):
     tol = 1e-12 if dt == torch.float64 else 1e-5
     assert O.rel_rmse(gp.cpu().numpy(), wp.cpu().numpy()) <= tol
     assert O.rel_rmse(dh, wh) <= tol
+
+
+@pytest.mark.parametrize("contiguous", [True, False])
+def test_tap_gradient_of_the_first_angles(torch, contiguous):
+    """Projections of the first angles only, in chunks, with a volume gradient of the
+    whole scan: dL/dh takes those angles' rows of the adjoint."""
+    from tomokvas_amd import diff
+
+    g = scan(40, 12, 9, 24, 20, 16, D=200.0, tau=0.1)
+    st = stages(g)
+    n = 7
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    p = torch.randn(st.sino_shape(n), device="cuda", generator=gen, dtype=torch.float64)
+    if not contiguous:
+        p = p.transpose(0, 1).contiguous().transpose(0, 1)
+    gvol = torch.randn(st.vol_shape, device="cuda", generator=gen, dtype=torch.float64)
+    say("tap gradient of the first angles")
+    _, dh = diff.backward(st, p, gvol, chunk=3, need_proj=False)
+    q = st.weight(p.contiguous().clone())
+    G = st.forward_project(gvol)[:, :n].contiguous()
+    ref = O.tap_gradient(ogeom(scan(40, 12, n, 24, 20, 16, D=200.0, tau=0.1)),
+                         q.cpu().numpy(), G.cpu().numpy())
+    assert O.rel_rmse(dh, ref) <= 1e-12
+    with pytest.raises(ValueError):
+        diff.backward(st, p, gvol, need_proj=False)

@@ -95,9 +95,9 @@ def backward(st: Stages, proj, gvol, chunk=None, need_proj=True, need_taps=True)
     dh = None
     if need_taps:
         dh = np.zeros(st.p, np.float64)
-        # q = W p is formed as the rows are read: a contiguous stack needs no copy
-        # and goes in one call
-        if proj.is_contiguous():
+        # q = W p is formed as the rows are read: a contiguous stack of all the angles
+        # needs no copy and goes in one call
+        if proj.is_contiguous() and proj.shape == gproj.shape:
             st.tap_gradient(proj.detach(), gproj, dh, weight=True)
         else:
             for a0 in range(0, nang, chunk):
