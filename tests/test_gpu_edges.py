@@ -116,3 +116,20 @@ def test_tap_gradient_of_the_first_angles(torch, contiguous):
     assert O.rel_rmse(dh, ref) <= 1e-12
     with pytest.raises(ValueError):
         diff.backward(st, p, gvol, need_proj=False)
+
+
+# zeros of both signs in one thread, in two lanes, waves and workgroups
+@pytest.mark.parametrize("at", [1, 4, 300, 2000, 5000, 40000, 99999])
+@pytest.mark.parametrize("first", [0.0, -0.0])
+def test_volume_range_keeps_the_sign_of_zero(torch, first, at):
+    """-0 is below +0, wherever either lies."""
+    import ctypes as C
+    L = _lib.load()
+    n = 100000
+    v = torch.full((n,), first, device="cuda")
+    v[at] = -first
+    mm = (C.c_double * 2)()
+    say(f"range of zeros, {-first} at {at}")
+    _lib.check(L.fdk_volume_minmax(C.c_void_p(v.data_ptr()), n, mm, None), "minmax")
+    assert (mm[0], mm[1]) == (0.0, 0.0)
+    assert np.signbit(mm[0]) and not np.signbit(mm[1])

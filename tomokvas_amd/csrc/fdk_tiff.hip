@@ -197,9 +197,9 @@ extern "C" int fdk_volume_minmax(const float *d_vol, size_t n, double *minmax, v
     if (e == hipSuccess) e = es;
     if (e != hipSuccess) return tkv::hip_fail(e, "minmax");
     float lo = part[0].x, hi = part[0].y;
-    for (unsigned k = 1; k < blocks; ++k) {
-        lo = std::min(lo, part[k].x);
-        hi = std::max(hi, part[k].y);
+    for (unsigned k = 1; k < blocks; ++k) {   // -0 below +0, as in the kernel
+        if (part[k].x < lo || (part[k].x == lo && std::signbit(part[k].x))) lo = part[k].x;
+        if (part[k].y > hi || (part[k].y == hi && !std::signbit(part[k].y))) hi = part[k].y;
     }
     if (lo > hi) return fail(FDK_ERR_INVALID_ARGUMENT, "minmax: no value that is not NaN");
     minmax[0] = lo;
