@@ -133,3 +133,23 @@ def test_volume_range_keeps_the_sign_of_zero(torch, first, at):
     _lib.check(L.fdk_volume_minmax(C.c_void_p(v.data_ptr()), n, mm, None), "minmax")
     assert (mm[0], mm[1]) == (0.0, 0.0)
     assert np.signbit(mm[0]) and not np.signbit(mm[1])
+
+
+@pytest.mark.parametrize("chunk", [None, 3])
+@pytest.mark.parametrize("store", [_lib.F32, _lib.F16])
+def test_forward_of_the_first_angles(torch, store, chunk):
+    """Projections of the first angles only give those angles' share of the volume."""
+    from tomokvas_amd import diff
+
+    g = scan(40, 12, 9, 24, 20, 16, D=200.0, tau=0.1)
+    st = stages(g)
+    n = 7
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    p = torch.randn(st.sino_shape(n), device="cuda", generator=gen)
+    say(f"forward of the first angles, storage {store}, chunk {chunk}")
+    got = diff.forward(st, p, storage=store, chunk=chunk)
+    q = torch.zeros(st.sino_shape(), device="cuda")
+    q[:, :n] = p
+    want = diff.forward(st, q, storage=store, chunk=chunk)
+    # the rows are transformed in other pairs
+    assert O.rel_rmse(got.cpu().numpy(), want.cpu().numpy()) <= (1e-3 if store == _lib.F16 else 1e-5)

@@ -59,8 +59,9 @@ def _slice(x, a0, n):
 
 
 def forward(st: Stages, proj, storage=_lib.F32, chunk=None):
-    """FDK of proj [Nv][Nang][Nu] with the context's filter; returns the volume.
-    FP64 input uses FP64 throughout; FP32 input is stored as `storage`."""
+    """FDK of proj [Nv][Nang][Nu] (or of the first angles) with the context's filter;
+    returns the volume.  FP64 input uses FP64 throughout; FP32 input is stored as
+    `storage`."""
     torch = _torch()
     nang = proj.shape[1]
     chunk = chunk or nang
@@ -81,7 +82,7 @@ def forward(st: Stages, proj, storage=_lib.F32, chunk=None):
         st.filter_into(src, y, weight=1, ang0=s0, maxabs=maxabs)   # per-projection max |y|
         st.pack_into(y, store, stack, scales, a0, maxabs)
         del y
-    return st.backproject(stack, store, scales)
+    return st.backproject(stack, store, scales, nang=nang)
 
 
 def backward(st: Stages, proj, gvol, chunk=None, need_proj=True, need_taps=True):
