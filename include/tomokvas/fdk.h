@@ -147,7 +147,8 @@ const float *fdk_device_volume(fdk_ctx *ctx);
  * with their own streams synchronised before fdk_calculate_reconstruction). */
 float *fdk_device_sinogram(fdk_ctx *ctx);
 /* Stage times of the last fdk_calculate_reconstruction in ms (device events):
- * [0] cosine weight + ramp filter, [1] pack to the storage type,
+ * [0] cosine weight + ramp filter, [1] pack to the storage type (FP16; the filter
+ * writes the other types' stored stack itself, so about 0),
  * [2] backprojection, [3] slab transfers + accumulation. */
 int fdk_get_stage_times(fdk_ctx *ctx, float *ms4);
 int fdk_get_geometry(fdk_ctx *ctx, int *ints8, float *floats12);

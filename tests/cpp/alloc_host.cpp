@@ -6,6 +6,7 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -14,6 +15,10 @@
 #include <string>
 #include <utility>
 #include <vector>
+
+namespace tkv {
+double engine_bytes_per_sample(int storage, int Nu);   // fdk_host.cpp
+}
 
 namespace {
 int launches = 0, allowed = -1, device = 0;   // allocations left (-1: any number)
@@ -72,6 +77,13 @@ void check(const char *what, bool ok)
 {
     std::printf("%s: %s\n", ok ? "ok" : "FAILED", what);
     if (!ok) good = false;
+}
+
+size_t bytes()
+{
+    size_t n = 0;
+    for (const auto &a : live) n += a.second.first;
+    return n;
 }
 
 fdk_ctx *context(int gpu, int storage)
@@ -163,6 +175,27 @@ int main(int argc, char **argv)
                                               into(p + rows / 4 - 1, 12, 12, FDK_BF16, p) == 0);
         check("no angles", fdk_filter_into(c, FDK_F32, p, 12, 0, 0, 0, -1, p + 1, nullptr, nullptr, nullptr) == FDK_OK);
         fdk_destroy(c);
+    } else if (mode == "budget") {
+        // what the reconstruction program charges for a projection is what the engine
+        // allocates for it (and for its angle's table entries)
+        for (int storage : {FDK_F32, FDK_F16, FDK_BF16, FDK_F16_PACKED})
+            for (int Nu : {40, 300, 1000}) {
+                size_t held[2] = {0, 0};
+                for (int i = 0; i < 2; ++i) {
+                    fdk_ctx *c = context(0, storage);
+                    const size_t before = bytes();
+                    if (fdk_set_sinogram_properties(c, nullptr, Nu, 0.f, 40 << i, 64, 0.f, 0.1f, 2000.f, 0.1f) ||
+                        fdk_initialize(c))
+                        check("initialized", false);
+                    held[i] = bytes();
+                    check("grown", held[i] > before);
+                    fdk_destroy(c);
+                }
+                const double per = (double)(held[1] - held[0]) / (40. * 64 * Nu);
+                const double charged = tkv::engine_bytes_per_sample(storage, Nu);
+                std::printf("storage %d Nu %d: %.4f bytes a sample, charged %.4f\n", storage, Nu, per, charged);
+                check("charged", std::fabs(per - charged) <= 0.02 + 100. / (64 * Nu));
+            }
     } else {
         std::printf("FAILED: unknown mode\n");
         return 2;

@@ -38,3 +38,8 @@ def test_storage_grows_on_the_context_s_device(exe):
 def test_filter_into_overlapping_buffers(exe):
     r = subprocess.run([exe, "overlap"], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr[-2000:]
+
+
+def test_angle_block_budget_is_what_the_engine_holds(exe):
+    r = subprocess.run([exe, "budget"], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr[-2000:]

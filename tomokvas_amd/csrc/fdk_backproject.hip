@@ -77,10 +77,7 @@ namespace tkv {
 
 static_assert(box_rows<64>() <= STACK_TAIL_ROWS, "stored stack tail shorter than a box");
 
-// Row pitch of the stored stack in samples: a multiple of 64 with at least
-// BOX_W + 4 zero samples after column Nu-1, so a staged box row that starts
-// inside the detector never leaves its own row.
-int stack_pitch(int Nu) { return ((Nu + BOX_W + 4 + 63) / 64) * 64; }
+static_assert(STACK_PAD >= BOX_W + BOX_ALIGN, "stored rows padded by less than a box");
 
 template <typename R>
 struct BPArgs {

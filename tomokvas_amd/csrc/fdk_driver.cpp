@@ -3,9 +3,10 @@
 // block, .bin/.siz output through the slab writer.
 //
 // Differences from the reference's main(), each deliberate:
-//  * the angle-block budget is what the engine needs on this GPU (filtered and
-//    stored stacks next to the projections, the whole volume resident), rounded
-//    down to whole projections so that no projection is left out of a block;
+//  * the angle-block budget is what the engine needs on this GPU (the stored stack
+//    and, for FP16 storage, the filtered projections next to the projections, the
+//    whole volume resident), rounded down to whole projections so that no
+//    projection is left out of a block;
 //  * the next angle block is read from disk on a loader thread while the engine
 //    works on the current one (two page-locked host buffers, so the upload runs
 //    at link speed);
@@ -289,19 +290,17 @@ extern "C" int fdk_reconstruct_file(const char *cra_path, const fdk_setting *set
         (unsigned long long)std::min(2 * ((rec_z + 7) / 8 + 32) + B, rec_z) * rec_x * rec_y *
         sizeof(float);
     const unsigned long long held_vol = streamed ? ring_bytes : vol_bytes;
-    // angle-block budget: the engine keeps the projections and the filtered
-    // stack in FP32 plus the stored stack (4, 2 or 2 bytes a sample), the
-    // volume (or its ring) and one collect slab; 10 % of the free memory is
-    // left spare (para_TC.cpp:65 leaves 10 % of free minus one slab for the
-    // projections)
+    // angle-block budget: the engine keeps the projections, the stored stack and
+    // for FP16 the filtered projections, the volume (or its ring) and one collect
+    // slab; 10 % of the free memory is left spare (para_TC.cpp:65 leaves 10 % of
+    // free minus one slab for the projections)
     long long budget = opt.angle_block_bytes;
     if (budget <= 0) {
         if (free_mem == 0)
             return fail(FDK_ERR_HIP, "driver: cannot query the free memory of GPU " +
                                          std::to_string(set->gpu_id) + " (no such device?)");
-        const double stored = opt.storage == FDK_F32 ? 4.0 : 2.0;
         const double usable = 0.9 * (double)free_mem - (double)held_vol - (double)slab_bytes;
-        budget = usable > 0 ? (long long)(usable * 4.0 / (8.0 + stored)) : 0;
+        budget = usable > 0 ? (long long)(usable * 4.0 / tkv::engine_bytes_per_sample(opt.storage, sx)) : 0;
     }
     budget = (long long)((unsigned long long)budget / proj_bytes * proj_bytes);
     if (budget < (long long)proj_bytes)

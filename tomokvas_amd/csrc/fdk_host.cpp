@@ -34,6 +34,13 @@ int padded_length(int Nu)
     return 2 * p;
 }
 
+double engine_bytes_per_sample(int storage, int Nu)
+{
+    const bool f16 = storage == FDK_F16 || storage == FDK_F16_PACKED;
+    const double sample = storage == FDK_F32 ? 4. : 2.;
+    return 4. + sample * stack_pitch(Nu) / Nu + (f16 ? 4. : 0.);
+}
+
 // CalcSinCos (kernel.cu:430-477): sin/cos of k*delta_f + rot evaluated in double.
 // The angle itself is formed in double from the float inputs (the reference
 // forms k*delta_f in float; the two differ by < Nang*dbeta*2^-24 rad).

@@ -129,7 +129,15 @@ struct BPLaunch {
 int launch_backproject(int store_dtype, const BPLaunch &a, hipStream_t st);
 BPShape bp_shape(int store_dtype, int Nx, int Ny, int Nz);
 int sample_bytes_of(int store_dtype);   // bytes of one stored sample
-int stack_pitch(int Nu);                // row pitch of the stored stack, samples
+// Row pitch of the stored stack in samples: a multiple of 64 with at least STACK_PAD
+// zero samples after column Nu-1, so a staged box row that starts inside the
+// detector never leaves its own row.
+constexpr int STACK_PAD = 68;
+inline int stack_pitch(int Nu) { return (Nu + STACK_PAD + 63) / 64 * 64; }
+// HBM bytes that an initialized engine holds per projection sample: the FP32
+// projections, the stored stack with its rows' padding and, for FP16, the filtered
+// projections
+double engine_bytes_per_sample(int storage, int Nu);
 constexpr int STACK_TAIL_ROWS = 128;    // spare rows after the last projection (>= box rows)
 
 struct FPLaunch {           // adjoint of the backprojector
