@@ -135,3 +135,45 @@ def test_taps_lie_inside_the_box(name, kernel):
         # voxels of four samples: boxes beyond the LDS tile beside staged ones (the
         # adjoint's hold this detector's 96 rows)
         assert kinds["beyond"] > 0, kinds
+
+
+def may_be_wide(g):
+    """may_be_wide() of fdk_adjoint.hip."""
+    across = 21.3 * g.scale
+    r = 0.5 * g.Nu + across
+    if g.D <= r:
+        return True
+    U = g.D / (g.D - r)
+    az_max = g.scale * (0.5 * g.Nz + abs(g.cz) + 64.)
+    return (63 * g.scale * U + az_max * across * U * U / g.D + 8. >= 128 or
+            across * (U + r * U * U / g.D) + 11. >= 64)
+
+
+@pytest.mark.parametrize("seed", range(40))
+def test_blocks_of_a_narrow_scan_are_narrow(seed):
+    """Where may_be_wide says no, no block with a column in the cylinder has a footprint
+    of 64 columns or 128 rows; the scans are drawn about the line between the two."""
+    from gpu_util import ogeom, scan
+
+    rng = np.random.default_rng(seed)
+    scale = float(rng.uniform(0.8, 2.1))
+    n = int(rng.integers(20, 120))
+    Nu = int(n * scale * rng.uniform(0.9, 1.5)) + 8
+    g = ogeom(scan(Nu, int(rng.integers(100, 400)), 13, n, n, int(rng.integers(30, 200)),
+                   D=float(Nu * np.exp(rng.uniform(np.log(0.7), np.log(20.)))), tau=0.1, scale=scale,
+                   cz=float(rng.uniform(-20, 20)), rot=float(rng.uniform(0, 1))))
+    ax, ay, az = [a.astype(f32) for a in O.axis_tables(g)]
+    az = np.concatenate([az, (az[-1] + (az[1] - az[0]) * np.arange(1, 129)).astype(f32)])
+    s64, c64 = O.sincos(g)
+    wide = False
+    for z0 in range(0, g.Nz, 64):
+        zs = az[z0], az[z0 + 63]
+        for y0 in range(0, g.Ny, 16):
+            for x0 in range(0, g.Nx, 16):
+                xs, ys = ax[x0:x0 + 16], ay[y0:y0 + 16]
+                if np.min(np.abs(xs)) ** 2 + np.min(np.abs(ys)) ** 2 >= 0.25 * g.Nu ** 2:
+                    continue
+                for b in range(g.Nang):
+                    wide = wide or footprint(f32(c64[b]), f32(s64[b]), (xs[0], xs[-1]),
+                                             (ys[0], ys[-1]), min(zs), max(zs), g, 64, 128)[2] < 0
+    assert may_be_wide(g) or not wide

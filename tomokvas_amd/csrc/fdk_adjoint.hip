@@ -178,18 +178,32 @@ __device__ __forceinline__ float lane_f32(float x, int lane)
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
 }
 
-// whether the footprints of all blocks of the 32 x 32 columns from (X0, Y0) are narrow
-__device__ inline bool narrow_angle(const FPArgs<float> &a, float c, float s, int X0, int Y0,
-                                    float azlo, float azhi)
-{
-    bool narrow = true;
-    for (int y = Y0; y < min(Y0 + 32, a.Ny); y += FP_BLOCK)
-        for (int x = X0; x < min(X0 + 32, a.Nx); x += FP_BLOCK)
-            narrow = footprint(c, s, a.ax[x], a.ax[min(x + FP_BLOCK, a.Nx) - 1], a.ay[y],
-                               a.ay[min(y + FP_BLOCK, a.Ny) - 1], azlo, azhi, a.cX, a.cZ, a.D,
-                               a.Nu, a.Nv, NARROW_H, NARROW_W).z >= 0 && narrow;
-    return narrow;
-}
+// first and last coordinate of each of the 2 x 2 blocks of 32 x 32 columns (blocks past
+// the volume repeat the last column's)
+struct BlockEdges {
+    float x0[2], x1[2], y0[2], y1[2];
+    __device__ __forceinline__ BlockEdges(const FPArgs<float> &a, int X0, int Y0)
+    {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            x0[h] = a.ax[min(X0 + h * FP_BLOCK, a.Nx - 1)];
+            x1[h] = a.ax[min(X0 + (h + 1) * FP_BLOCK, a.Nx) - 1];
+            y0[h] = a.ay[min(Y0 + h * FP_BLOCK, a.Ny - 1)];
+            y1[h] = a.ay[min(Y0 + (h + 1) * FP_BLOCK, a.Ny) - 1];
+        }
+    }
+    // whether the footprints of all blocks are narrow
+    __device__ inline bool narrow(const FPArgs<float> &a, float c, float s, float azlo,
+                                  float azhi) const
+    {
+        bool all = true;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            all = footprint(c, s, x0[q & 1], x1[q & 1], y0[q >> 1], y1[q >> 1], azlo, azhi, a.cX,
+                            a.cZ, a.D, a.Nu, a.Nv, NARROW_H, NARROW_W).z >= 0 && all;
+        return all;
+    }
+};
 
 // Lanes run along z: in each splat instruction the 64 lanes of a wave are the
 // 64 slices of one (x, y) column, so their taps share the column and sit on
@@ -272,14 +286,14 @@ __global__ void __launch_bounds__(FP_THREADS) fp_lds_kernel(FPArgs<float> a)
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int z0 = zr * FP_ZR;
     const int xa = tx * T, ya = ty * T;
-    const int X0 = xa & ~31, Y0 = ya & ~31;
     const float az0 = a.az[z0], az1 = a.az[z0 + FP_ZR - 1];
     const float azlo = fminf(az0, az1), azhi = fmaxf(az0, az1);
+    const BlockEdges edges(a, xa & ~31, ya & ~31);
     if (a.wide) {
         // any angle of this kernel's kind?
         bool mine = false;
         for (int b = b0 + threadIdx.x; b < b1; b += FP_THREADS)
-            mine = mine || narrow_angle(a, a.ang[2 * b], a.ang[2 * b + 1], X0, Y0, azlo, azhi) != WIDE;
+            mine = mine || edges.narrow(a, a.ang[2 * b], a.ang[2 * b + 1], azlo, azhi) != WIDE;
         if (!__syncthreads_or(mine)) return;
     }
 
@@ -497,14 +511,13 @@ __global__ void __launch_bounds__(FP_THREADS) fp_lds_kernel(FPArgs<float> a)
                     const float c = a.ang[2 * (b + lane)], s = a.ang[2 * (b + lane) + 1];
                     int4 q = footprint(c, s, cx0, cx1, cy0, cy1, azlo, azhi, a.cX, a.cZ, a.D, a.Nu,
                                        a.Nv, H, W);
-                    const bool narrow = narrow_angle(a, c, s, X0, Y0, azlo, azhi);
-                    if (WIDE) {
-                        if (narrow) q.z = 0;
-                        else if (q.z > 0 && (direct || steep)) q.z = -1;
-                    } else if (!narrow && a.wide) {
-                        q.z = 0;
-                    } else if (q.z != 0 && (direct || !narrow)) {
-                        q.z = -1;
+                    const bool narrow = !a.wide || edges.narrow(a, c, s, azlo, azhi);
+                    if (narrow == WIDE) {
+                        q.z = 0;          // the other kernel's
+                    } else if (WIDE) {
+                        if (q.z > 0 && (direct || steep)) q.z = -1;
+                    } else if (direct) {
+                        if (q.z != 0) q.z = -1;
                     } else if (q.z < 0) {
                         q = footprint(c, s, cx0, cx1, cy0, cy1, azlo, azhi, a.cX, a.cZ, a.D, a.Nu,
                                       a.Nv, FP_H2, FP_W2);
@@ -675,17 +688,17 @@ static int fp_splits(long long tiles, int nang)
     return (int)best;
 }
 
-// Whether a block's footprint may be wide somewhere: its rows and columns at the
-// cylinder's edge nearest to the source (U varies over a block, 15 sqrt 2 voxels
-// across, by at most U^2/D per unit of S).  Too low a figure costs time only: the
-// first kernel then splats such an angle straight into HBM.
+// Whether the footprint of a block with a column in the cylinder may be wide: bounds
+// on its rows and columns at the cylinder's edge nearest to the source, with a sample
+// to spare (U varies over a block, 15 sqrt 2 voxels across, by at most U^2/D per unit
+// of S; a box has 7 rows and 10 columns beyond the span of the block's taps).
 static bool may_be_wide(const FPLaunch &L)
 {
     const double across = 21.3 * L.scale, r = std::sqrt(L.maskR2) + across;
     if (L.D <= r) return true;
     const double U = L.D / (L.D - r);
     const double rows = (FP_ZR - 1) * L.scale * U + L.az_max * across * U * U / L.D + 8.;
-    const double cols = across * (U + r * U * U / L.D) + 9.;
+    const double cols = across * (U + r * U * U / L.D) + 11.;
     return rows >= NARROW_H || cols >= NARROW_W;
 }
 
