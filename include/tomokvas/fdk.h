@@ -95,7 +95,9 @@ int fdk_set_reconstruction_properties(fdk_ctx *ctx, int Nx, float cx, int Ny, fl
                                       int Nz, float cz, float rot);
 int fdk_set_scale_xyz(fdk_ctx *ctx, float scale);                  /* SetScaleXYZ     */
 /* extensions: ramp filter choice (default Ram-Lak, as the reference) and the
- * storage type of the filtered stack (default FDK_F32) */
+ * storage type of the filtered stack (default FDK_F32; on an initialized context
+ * the stack grows as needed, and if it can't be had the old type stays and the
+ * context needs fdk_initialize again) */
 int fdk_set_filter(fdk_ctx *ctx, int kind, const double *taps, int ntaps);
 int fdk_set_storage(fdk_ctx *ctx, int dtype);
 /* extension: volume residency (default FDK_VOLUME_RESIDENT), set before

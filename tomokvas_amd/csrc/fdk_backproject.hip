@@ -777,24 +777,26 @@ static int native_zrun(int dtype)
     }
 }
 
-// The long z-runs (slices per thread, TKV_BP_ZR_*) spread a column's set-up over the most updates and read each
-// box row for the most slices, but a volume of few blocks leaves CUs idle, or ends
-// on a mostly idle last wave.  So a smaller volume takes runs of 16 slices, and one
+// The long z-runs (slices per thread, TKV_BP_ZR_*) spread a column's set-up over the
+// most updates and read each box row for the most slices, but a volume of few blocks
+// leaves CUs idle, or ends on a mostly idle last wave.  So a smaller volume takes runs of 16 slices, and one
 // whose blocks still don't fill the 256 CUs has 2 or 4 groups of 256 threads per
 // block, each gathering every 2nd or 4th angle from a box of its own; their sums
-// meet in LDS.  By blocks of 16^3 voxels; us for 32-slice (FP32: 24) runs, runs of
-// 16 with 1, 2, 4 groups, runs of 8 with 4 groups (before a slice's reads were
-// issued ahead, which takes another 3 to 6 % off most):
-//      8  32^3, 36 angles              60    45    33    30    22
-//     64  64^3, 90 angles             142   100    72    61    44
-//    108  96^2 x 40, 120, FP16        232   145    98    79    54
-//    180  96^2 x 80, 150, BF16        292   159   114    94   129
-//    512  128^3, 180                  320   224   186   218   284
-//   1000  160^2 x 150, 240, BF16      557   441   446   567   731
-//   1690  203^2 x 157, 251            741   689   792   951  1313
-//   4096  256^3, 360                 2026  1939  2410  3003  4013
-//   7600  320^2 x 300, 360, BF16     3519  3221  3594  5539  7860
-//  15625  400^3, 400                 7403  7543  9556 12319 17095
+// meet in LDS.  By blocks of 16^3 voxels; us for the long runs, runs of 16 with 1, 2, 4
+// groups, runs of 8 with 4 groups, FP32 / FP16 (BF16 like FP16; packed FP16 within 10 %
+// at the shapes taken):
+//       8  32^3, 36                      57 / 57        34 / 35        26 / 26        24 / 24        17 / 18
+//      64  64^3, 90                    133 / 133        83 / 85        60 / 61        51 / 52        37 / 37
+//     108  96^2 x 40, 120              180 / 220      133 / 136        90 / 90        70 / 70        42 / 43
+//     180  96^2 x 80, 150              223 / 278      139 / 142        97 / 98        78 / 79      101 / 103
+//     512  128^3, 180                  302 / 269      198 / 201      160 / 161      184 / 186      239 / 246
+//    1000  160^2 x 150, 240            498 / 528      406 / 407      438 / 402      508 / 516      636 / 655
+//    1560  203 x 190 x 157, 251        713 / 676      562 / 556      643 / 574      769 / 782    1056 / 1090
+//    4096  256^3, 360                1907 / 1828    1817 / 1769    2125 / 1881    2638 / 2690    3606 / 3708
+//    7600  320^2 x 300, 360          3267 / 3355    3212 / 3104    3886 / 3390    4878 / 4967    6652 / 6844
+//   15625  400^3, 400                6924 / 7004    7112 / 6780    8740 / 7567  11195 / 11413  15583 / 16031
+// One rule serves all types, where a single one could do better: FP32 by 8 % with one
+// group at 1000 blocks, 16-bit samples by 3 % with runs of 16 at 15625.
 // Taken from the whole volume and from neither the angles nor the slices of one
 // launch, so that a volume in z-chunks gets the sums of one launch.  (FP64 gathers
 // from HBM without boxes and keeps its runs of 8.)

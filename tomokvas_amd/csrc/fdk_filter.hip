@@ -727,8 +727,9 @@ __global__ void __launch_bounds__(PL::BLOCK)
     cpx<R> acc[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) acc[e] = {0, 0};
-    // row pairs [first, pairs) of all rows; the bound is the same for every thread of the workgroup (the passes'
-    // barriers are workgroup-wide); a transform past the last pair adds zeros
+    // row pairs [first, pairs) of all rows; the bound is the same for every thread of
+    // the workgroup (the passes' barriers are workgroup-wide); a transform past the
+    // last pair adds zeros
     for (long long pr0 = first + (long long)blockIdx.x * PL::NT; pr0 < pairs;
          pr0 += (long long)gridDim.x * PL::NT) {
         const long long pr = pr0 + f;

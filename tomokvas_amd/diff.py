@@ -14,8 +14,9 @@ BP: the backprojector (kernel.cu:68-177).  The adjoints are hand-written:
 
 With ``chunk`` set, neither pass holds a filtered or weighted copy of the
 whole stack: the forward pass filters and packs ``chunk`` projections at a time
-into the stored stack, and the backward pass recomputes q = W p as it is read.  The backward pass forward-projects all angles
-at once straight into the gradient buffer (one read of the volume gradient).
+into the stored stack, and the backward pass recomputes q = W p as it is read.  The
+backward pass forward-projects all angles at once straight into the gradient buffer
+(one read of the volume gradient).
 """
 from __future__ import annotations
 
